@@ -8,17 +8,19 @@
 //                   six directional sweeps of the Eikonal update
 //                   update_from_neighbor (level_set.py:88-112).
 //
-// Sweeps: one thread owns one grid line along the sweep axis and walks it in
-// the sweep direction, so the cells behind it on the line are already updated
-// and the ones ahead are not, as in the reference's serial inner loop.  The
-// reference runs the lines in parallel and reads the neighbouring lines while
-// they change (the result depends on thread timing); here the neighbouring
-// lines are read from a copy taken before the sweep, which makes the result
-// deterministic.  Each axis is swept over its own extent (the reference bounds
-// the axis-0 sweeps by res[1], level_set.py:297-303/323-327, which only
-// differs on non-square grids).
+// Sweeps: a grid line along the sweep axis is walked in the sweep direction,
+// so the cells behind it on the line are already updated and the ones ahead
+// are not, as in the reference's serial inner loop.  The reference runs the
+// lines in parallel and reads the neighbouring lines while they change (the
+// result depends on thread timing); here the neighbouring lines are read as
+// they were before the sweep (a sweep reads one array and writes another),
+// which makes the result deterministic.  Each axis is swept over its own
+// extent (the reference bounds the axis-0 sweeps by res[1],
+// level_set.py:297-303/323-327, which only differs on non-square grids).
 #include <hip/hip_runtime.h>
 #include <math.h>
+
+#include <type_traits>
 
 #include "../../include/mgpcg.h"
 #include "mgpcg_common.h"
@@ -82,95 +84,319 @@ __global__ void k_init_boundary(Grid g, int8_t* __restrict__ ct) {
     if (I[a] == 0 || I[a] + 1 == g.n[a]) ct[t] = MG_SOLID;
 }
 
+// What a sweep needs of a cell besides its distance, in one byte (the
+// caller's `fixed` work array): bit 0 = fixed by target_surface, bits 1-2 =
+// sign(phi) + 1.
+__device__ __forceinline__ float code_sign(int code) { return (float)((code >> 1) - 1); }
+
 // target_surface (level_set.py:66-86): cells with a sign change to a face
 // neighbour take the signed distance estimate sign(phi) * theta * dx of the
-// closest crossing and are fixed; the others start at 1e20.
-__global__ void k_target_surface(Grid g, const float* __restrict__ phi, float dx,
-                                 float* __restrict__ tmp, int8_t* __restrict__ fixed) {
+// closest crossing and are fixed; the others start at 1e20.  Every neighbour
+// is loaded before any is used (a missing one reads the cell itself, which
+// has no sign change to it).  256^3: 141 us with a wait per neighbour -> 73 us,
+// where the 9 B a cell reads and writes would take 32.
+template <int DIM>
+__global__ void __launch_bounds__(LB) k_target_surface(Grid g, const float* __restrict__ phi,
+                                                       float dx, float* __restrict__ tmp,
+                                                       int8_t* __restrict__ code) {
   const long t = (long)blockIdx.x * LB + threadIdx.x;
   if (t >= g.cells()) return;
   int I[3];
   coords(g, t, I);
   const float pi = phi[t];
+  float pj[DIM][2];
+#pragma unroll
+  for (int k = 0; k < DIM; ++k) {
+    pj[k][0] = phi[I[k] > 0 ? t - g.st[k] : t];
+    pj[k][1] = phi[I[k] + 1 < g.n[k] ? t + g.st[k] : t];
+  }
+  const float si = sgnf(pi);
   bool change = false;
   float est = 1e20f;
-  for (int k = 0; k < g.dim; ++k) {
-    for (int s = -1; s <= 1; s += 2) {
-      const int j = I[k] + s;
-      if (j < 0 || j >= g.n[k]) continue;
-      const float pj = phi[t + s * g.st[k]];
-      if (sgnf(pi) != sgnf(pj)) {
-        const float th = pi / (pi - pj);
-        const float est0 = sgnf(pi) * th * dx;
+#pragma unroll
+  for (int k = 0; k < DIM; ++k)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      if (si != sgnf(pj[k][h])) {
+        const float th = pi / (pi - pj[k][h]);
+        const float est0 = si * th * dx;
         est = fabsf(est0) < fabsf(est) ? est0 : est;
         change = true;
       }
-    }
-  }
-  tmp[t] = change ? est : 1e20f;
-  fixed[t] = change ? 1 : 0;
+  tmp[t] = est;
+  code[t] = (int8_t)((change ? 1 : 0) | (((int)si + 1) << 1));
 }
 
 struct EikonalConsts {
   float dx, two_dx2, dx2, half, third;
 };
 
-// update_from_neighbor (level_set.py:88-112); along axis `ax` the values come
-// from the live array (the sweeping thread's own line), across from `snap`.
-__device__ float eikonal(const Grid& g, const int* I, long t, int ax, const float* live,
-                         const float* snap, const EikonalConsts& c) {
-  float nb[3] = {0.0f, 0.0f, 0.0f};
-  for (int k = 0; k < g.dim; ++k) {
-    const float* f = (k == ax) ? live : snap;
-    const long o = g.st[k];
-    if (I[k] == 0 || (I[k] < g.n[k] - 1 && fabsf(f[t + o]) < fabsf(f[t - o])))
-      nb[k] = fabsf(f[t + o]);
-    else
-      nb[k] = fabsf(f[t - o]);
-  }
-  for (int i = 0; i < g.dim - 1; ++i)
-    for (int j = 0; j < g.dim - 1 - i; ++j)
-      if (nb[j] > nb[j + 1]) {
-        const float x = nb[j];
-        nb[j] = nb[j + 1];
-        nb[j + 1] = x;
-      }
-  float d = nb[0] + c.dx;
-  if (d > nb[1]) {
-    const float df = nb[1] - nb[0];
-    d = c.half * (nb[0] + nb[1] + sqrtf(c.two_dx2 - df * df));
-    if (g.dim == 3 && d > nb[2]) {
-      const float s = nb[0] + nb[1] + nb[2];
-      const float q = nb[0] * nb[0] + nb[1] * nb[1] + nb[2] * nb[2] - c.dx2;
-      d = c.third * (s + sqrtf(fmaxf(0.0f, s * s - 3.0f * q)));
-    }
-  }
-  return d;
+// The smaller and the larger of two magnitudes: their bit patterns order as
+// they do, and an integer compare needs no quieting of NaNs first.
+__device__ __forceinline__ float nearer(float a, float b) {
+  const uint32_t x = __float_as_uint(a) & 0x7fffffffu, y = __float_as_uint(b) & 0x7fffffffu;
+  return __uint_as_float(x < y ? x : y);
+}
+__device__ __forceinline__ float lesser(float a, float b) {
+  const uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+  return __uint_as_float(x < y ? x : y);
+}
+__device__ __forceinline__ float larger(float a, float b) {
+  const uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+  return __uint_as_float(x < y ? y : x);
 }
 
-// One directional sweep: a thread per line along `ax`, dir = +1 / -1.
-__global__ void k_sweep(Grid g, int ax, int dir, const float* __restrict__ phi,
-                        const float* __restrict__ snap, float* __restrict__ tmp,
-                        const int8_t* __restrict__ fixed, EikonalConsts c) {
-  const long nlines = g.cells() / g.n[ax];
-  const long line = (long)blockIdx.x * LB + threadIdx.x;
-  if (line >= nlines) return;
-  // the line's coordinates on the other axes (C order over them)
-  int I[3] = {0, 0, 0};
-  long r = line;
-  for (int a = g.dim - 1; a >= 0; --a) {
-    if (a == ax) continue;
-    I[a] = (int)(r % g.n[a]);
-    r /= g.n[a];
+// sqrtf, correctly rounded, for an argument that is 0, +inf or at least
+// 2^-96: the hardware's root (within 1 ulp) and Tuckerman's test of its two
+// neighbours (s is the rounded root of x when s (s - ulp) < x <= s (s + ulp)).
+// The compiler's sqrtf spends six more instructions on scaling smaller
+// arguments; the sweeps below are bound by the instructions of their chains.
+__device__ __forceinline__ float root(float x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const float s = __builtin_amdgcn_sqrtf(x);
+  const float below = __uint_as_float(__float_as_uint(s) - 1u);
+  const float above = __uint_as_float(__float_as_uint(s) + 1u);
+  const float r = __builtin_fmaf(-below, s, x) <= 0.0f ? below : s;
+  return __builtin_fmaf(-above, s, x) > 0.0f ? above : r;
+#else
+  return sqrtf(x);
+#endif
+}
+
+// update_from_neighbor (level_set.py:88-112) from the nearer neighbour `a`
+// along the line and the nearer ones across it, m1 <= m2 (2D: m1 alone).
+// The three are merged in order (no distance is ever NaN: target_surface and
+// the sweeps store a value only where it compares less than another one), and
+// every candidate is formed, so nothing but the choice waits for a compare.
+// ROOT: both roots' arguments are in root's range where their result counts.
+template <int DIM, bool ROOT>
+__device__ __forceinline__ float eikonal(float a, float m1, float m2, const EikonalConsts& c) {
+  auto rt = [](float x) { return ROOT ? root(x) : sqrtf(x); };
+  const float n0 = lesser(a, m1);
+  const float n1 = DIM == 3 ? lesser(larger(a, m1), m2) : larger(a, m1);
+  const float d1 = n0 + c.dx;
+  const float df = n1 - n0;
+  float d2 = c.half * (n0 + n1 + rt(c.two_dx2 - df * df));
+  if (DIM == 3) {
+    const float n2 = larger(a, m2);
+    const float s = n0 + n1 + n2;
+    const float q = n0 * n0 + n1 * n1 + n2 * n2 - c.dx2;
+    const float d3 = c.third * (s + rt(fmaxf(0.0f, s * s - 3.0f * q)));
+    d2 = d2 > n2 ? d3 : d2;
   }
-  const int n = g.n[ax];
-  for (int step = 0; step < n; ++step) {
-    I[ax] = dir > 0 ? step : n - 1 - step;
-    long t = 0;
-    for (int a = 0; a < g.dim; ++a) t += I[a] * g.st[a];
-    if (fixed[t]) continue;
-    const float d = eikonal(g, I, t, ax, tmp, snap, c);
-    if (fabsf(d) < fabsf(tmp[t])) tmp[t] = d * sgnf(phi[t]);
+  return d1 > n1 ? d2 : d1;
+}
+
+// Workgroup w of n works on part xcd_part(w, n): workgroups go to the 8 XCDs
+// in turn, so this gives each XCD a contiguous range of parts, whose shared
+// neighbour lines then meet in its L2.
+__device__ __forceinline__ int xcd_part(int w, int n) {
+  const int q = n / 8, r = n % 8, x = w % 8;
+  return x * q + min(x, r) + w / 8;
+}
+
+// One directional sweep along axis AX.  A line is a serial chain, each cell
+// waiting for the one before it, and a wave's chain is bound by the
+// instructions it issues (4 cycles each, one wave per SIMD), so everything
+// that does not wait is taken off it: a workgroup has SW_LINES lines in
+// chunks of SW_STEPS steps; its last four waves read a chunk's cells and the
+// lines across, coalesced, and leave in one of two LDS buffers each cell's
+// distance and its two sorted cross neighbours, while the first wave walks
+// the other buffer, a lane per line, on magnitudes alone.  The walked
+// magnitudes replace the cross neighbours, and the filling waves sign and
+// store them, coalesced, before that buffer is filled again (each thread the
+// places it fills).  On the contiguous axis a line's steps are consecutive in
+// LDS (17 words a line: no bank conflicts for the walk), on the others the
+// lines of a step.  37 KB of LDS: four workgroups per CU.
+// A sweep at 256^3: 77 us on the contiguous axis, 75 us on the others, bound
+// by issue (one walking and four filling waves per SIMD); a thread per line
+// on global memory, with a copy of the array before it, took 1390 and 600 us.
+// At 131 x 97 x 150, 20-27 us, bound by the chain (about 150 ns a step in 3D,
+// 70 ns in 2D).
+constexpr int SW_LINES = 64;
+constexpr int SW_STEPS = 16;
+constexpr int SW_FILL = 256;
+constexpr int SW_THREADS = 64 + SW_FILL;
+constexpr int SW_MINE = SW_LINES * SW_STEPS / SW_FILL;  // places per filling thread
+constexpr int SW_WORDS = SW_LINES * (SW_STEPS + 1);     // one step more: the chunk's next cell
+template <int DIM, int AX, bool ROOT, typename IX>
+__global__ void __launch_bounds__(SW_THREADS, 5) k_sweep(Grid g, int dir,
+                                                      const float* __restrict__ src,
+                                                      float* __restrict__ dst,
+                                                      const int8_t* __restrict__ code,
+                                                      EikonalConsts c) {
+  constexpr bool CONTIG = AX == DIM - 1;
+  // the axes across: B, and in 3D A
+  constexpr int B = CONTIG ? DIM - 2 : DIM - 1, A = DIM == 2 ? B : (AX == 0 ? 1 : 0);
+  __shared__ float own[2][SW_WORDS];   // the cells' distances, signed
+  __shared__ float thr[2][SW_WORDS];   // |distance| to undercut: 0 where fixed
+  __shared__ float m1[2][SW_WORDS];    // nearer neighbours across; the walked magnitudes
+  __shared__ float m2[2][SW_WORDS];
+  __shared__ int8_t cd[2][SW_WORDS];   // cell codes
+  // chunk ch has an unfixed cell of sign 0 (its distance becomes 0): slot
+  // ch & 3, cleared two chunks before it is filled
+  __shared__ int flat[4];
+  auto place = [](int line, int step) {
+    return CONTIG ? line * (SW_STEPS + 1) + step : step * SW_LINES + line;
+  };
+  const int n = g.n[AX];
+  const long nlines = g.cells() / n;
+  const long line0 = (long)xcd_part((int)blockIdx.x, (int)gridDim.x) * SW_LINES;
+  const int nchunks = (n + SW_STEPS - 1) / SW_STEPS;
+  const int tid = (int)threadIdx.x;
+  // filling thread f's places i: line fl + i * FL, step fs + i * FS of a chunk
+  // (the walking wave computes them too and does not use them)
+  constexpr int FL = CONTIG ? SW_FILL / SW_STEPS : 0, FS = CONTIG ? 0 : SW_FILL / SW_LINES;
+  const int f = tid - 64;
+  const int fl = CONTIG ? max(f, 0) / SW_STEPS : max(f, 0) & (SW_LINES - 1);
+  const int fs = CONTIG ? f & (SW_STEPS - 1) : max(f, 0) / SW_LINES;
+  // its lines' first cells in sweep order (a line past the last one reads the
+  // last one and is not stored) and the offsets to the lines across; on a side
+  // without one the other side's line is read twice (every axis has at least
+  // two cells), which leaves the nearer of the two the same
+  constexpr int NL = CONTIG ? SW_MINE : 1;
+  const IX st = (IX)(dir > 0 ? g.st[AX] : -g.st[AX]), stb = (IX)g.st[B], sta = (IX)g.st[A];
+  IX first[NL], obl[NL], obh[NL], oal[NL], oah[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const long line = min(line0 + fl + i * FL, nlines - 1);
+    // the line's coordinates on B and A: C order over those axes
+    constexpr int SLOW = DIM == 2 ? B : (A < B ? A : B), FAST = DIM == 2 ? B : (A < B ? B : A);
+    const int is = DIM == 3 ? (int)(line / g.n[FAST]) : 0;
+    const int ifa = (int)(line - (long)is * g.n[FAST]);
+    first[i] = (IX)((DIM == 3 ? is * g.st[SLOW] : 0) + ifa * g.st[FAST] +
+                    (dir > 0 ? 0 : (n - 1) * g.st[AX]));
+    const int ib = FAST == B ? ifa : is, ia = FAST == B ? is : ifa;
+    obl[i] = ib > 0 ? -stb : stb;
+    obh[i] = ib + 1 < g.n[B] ? stb : -stb;
+    oal[i] = ia > 0 ? -sta : sta;
+    oah[i] = ia + 1 < g.n[A] ? sta : -sta;
+  }
+  auto at = [](auto* base, IX i) {
+    if constexpr (sizeof(IX) == 4) return ldgi(base, i);
+    else return ldg(base + i);
+  };
+  // A chunk that reaches the line's end (`tail`) clamps its steps there; the
+  // others, and workgroups with all their lines, do without any test.
+  const bool lines = line0 + SW_LINES <= nlines;
+  auto tail = [&](int chunk) { return (chunk + 1) * SW_STEPS >= n; };
+  auto store_t = [&](int chunk, auto test) {
+    const int b = chunk & 1, s0 = chunk * SW_STEPS + fs;
+#pragma unroll
+    for (int i = 0; i < SW_MINE; ++i) {
+      const int s = s0 + i * FS, w = place(fl + i * FL, fs + i * FS);
+      if (decltype(test)::value && (line0 + fl + i * FL >= nlines || s >= n)) continue;
+      const float mag = m1[b][w], was = own[b][w];
+      const float v = mag < fabsf(was) ? mag * code_sign(cd[b][w]) : was;
+      const IX t = first[CONTIG ? i : 0] + s * st;
+      if constexpr (sizeof(IX) == 4) stgi(dst, t, v);
+      else stg(dst + t, v);
+    }
+  };
+  auto store = [&](int chunk) {
+    if (lines && !tail(chunk)) store_t(chunk, std::false_type());
+    else store_t(chunk, std::true_type());
+  };
+  // a chunk's values on their way to LDS: loaded a chunk ahead, so that their
+  // latency passes behind the walk of the chunk between
+  float v[SW_MINE], nx[SW_MINE], bl[SW_MINE], bh[SW_MINE], al[SW_MINE], ah[SW_MINE];
+  int cv[SW_MINE];
+  auto fetch_t = [&](int chunk, auto clamp) {
+    const int s0 = chunk * SW_STEPS + fs;
+#pragma unroll
+    for (int i = 0; i < SW_MINE; ++i) {
+      const int l = CONTIG ? i : 0;
+      const int s = decltype(clamp)::value ? min(s0 + i * FS, n - 1) : s0 + i * FS;
+      const IX t = first[l] + s * st;
+      v[i] = at(src, t);
+      bl[i] = at(src, t + obl[l]);
+      bh[i] = at(src, t + obh[l]);
+      if (DIM == 3) {
+        al[i] = at(src, t + oal[l]);
+        ah[i] = at(src, t + oah[l]);
+      }
+      cv[i] = at(code, t);
+      // the chunk's last step carries the next cell of the line too
+      if (CONTIG || i == SW_MINE - 1)
+        nx[i] = at(src, !decltype(clamp)::value || s + 1 < n ? t + st : t);
+    }
+  };
+  auto fetch = [&](int chunk) {
+    if (tail(chunk)) fetch_t(chunk, std::true_type());
+    else fetch_t(chunk, std::false_type());
+  };
+  auto put = [&](int chunk) {
+    const int b = chunk & 1, s0 = chunk * SW_STEPS + fs;
+    bool zero = false;
+#pragma unroll
+    for (int i = 0; i < SW_MINE; ++i) {
+      const int step = fs + i * FS, w = place(fl + i * FL, step);
+      const float mb = nearer(bl[i], bh[i]);
+      const float ma = DIM == 3 ? nearer(al[i], ah[i]) : INFINITY;
+      const bool fixed = (cv[i] & 1) != 0;
+      // past the line's end: no neighbour ahead
+      own[b][w] = s0 + i * FS < n ? v[i] : INFINITY;
+      if ((CONTIG || i == SW_MINE - 1) && step == SW_STEPS - 1)
+        own[b][place(fl + i * FL, SW_STEPS)] = s0 + i * FS + 1 < n ? nx[i] : INFINITY;
+      thr[b][w] = fixed ? 0.0f : fabsf(v[i]);
+      m1[b][w] = DIM == 3 ? lesser(mb, ma) : mb;
+      if (DIM == 3) m2[b][w] = larger(mb, ma);
+      cd[b][w] = (int8_t)cv[i];
+      zero = zero || cv[i] == 2;  // not fixed, sign 0
+    }
+    if (zero) flat[chunk & 3] = 1;
+  };
+  // the walked magnitudes of chunk buffer b (steps past the line's end walk
+  // over what the buffer holds, and are not stored)
+  float prev = INFINITY;
+  auto walk = [&](int b, auto zeros) {
+    float nx[SW_STEPS], lim[SW_STEPS], a1[SW_STEPS], a2[SW_STEPS];
+    const float here = own[b][place(tid, 0)];
+#pragma unroll
+    for (int u = 0; u < SW_STEPS; ++u) {
+      nx[u] = own[b][place(tid, u + 1)];
+      lim[u] = thr[b][place(tid, u)];
+      a1[u] = m1[b][place(tid, u)];
+      a2[u] = DIM == 3 ? m2[b][place(tid, u)] : INFINITY;
+    }
+#pragma unroll
+    for (int u = 0; u < SW_STEPS; ++u) {
+      const float was = fabsf(u == 0 ? here : nx[u - 1]);
+      float d = eikonal<DIM, ROOT>(nearer(prev, nx[u]), a1[u], a2[u], c);
+      const bool less = d < lim[u];
+      if (decltype(zeros)::value) d = d * fabsf(code_sign(cd[b][place(tid, u)]));
+      prev = less ? d : was;
+      m1[b][place(tid, u)] = prev;
+    }
+  };
+  if (tid < 4) flat[tid] = 0;
+  // Both sides of the branch, each taken by whole waves, pass the same
+  // barriers: one here, one before every chunk, one after the last.  (Two
+  // loops rather than one keep the filling waves' values out of the walking
+  // wave's registers.)
+  __syncthreads();
+  if (f >= 0) {
+    fetch(0);
+    put(0);
+    fetch(1);
+    for (int ch = 0; ch < nchunks; ++ch) {
+      __syncthreads();  // buffer ch & 1 is filled, the other one walked
+      if (ch > 0) store(ch - 1);
+      if (ch + 1 < nchunks) {
+        put(ch + 1);
+        fetch(ch + 2);
+      }
+    }
+    __syncthreads();
+    store(nchunks - 1);
+  } else {
+    for (int ch = 0; ch < nchunks; ++ch) {
+      __syncthreads();
+      if (tid == 0) flat[(ch + 2) & 3] = 0;
+      if (flat[ch & 3]) walk(ch & 1, std::true_type());
+      else walk(ch & 1, std::false_type());
+    }
+    __syncthreads();
   }
 }
 
@@ -246,6 +472,39 @@ __global__ void k_copy8(long n, const int8_t* __restrict__ src, int8_t* __restri
 
 inline unsigned nblk(long n) { return (unsigned)((n + LB - 1) / LB); }
 
+template <int DIM, int AX>
+void sweep_t(hipStream_t s, const Grid& g, int dir, const float* src, float* dst,
+             const int8_t* code, const EikonalConsts& c) {
+  const long nlines = g.cells() / g.n[AX];
+  const dim3 grid((unsigned)((nlines + SW_LINES - 1) / SW_LINES));
+  // The roots' arguments are sums and products of distances rounded to 24
+  // bits: 0 or at least dx^2 2^-24 where their result counts, so above root's
+  // 2^-96 for every dx but the smallest.  32-bit offsets reach 2^30 cells.
+  if (c.dx < 0x1p-32f)
+    hipLaunchKernelGGL((k_sweep<DIM, AX, false, long>), grid, dim3(SW_THREADS), 0, s, g, dir, src,
+                       dst, code, c);
+  else if (g.cells() > (1l << 30))
+    hipLaunchKernelGGL((k_sweep<DIM, AX, true, long>), grid, dim3(SW_THREADS), 0, s, g, dir, src,
+                       dst, code, c);
+  else
+    hipLaunchKernelGGL((k_sweep<DIM, AX, true, int>), grid, dim3(SW_THREADS), 0, s, g, dir, src,
+                       dst, code, c);
+}
+
+void sweep(hipStream_t s, const Grid& g, int ax, int dir, const float* src, float* dst,
+           const int8_t* code, const EikonalConsts& c) {
+  if (g.dim == 2) {
+    if (ax == 0) sweep_t<2, 0>(s, g, dir, src, dst, code, c);
+    else sweep_t<2, 1>(s, g, dir, src, dst, code, c);
+  } else if (ax == 0) {
+    sweep_t<3, 0>(s, g, dir, src, dst, code, c);
+  } else if (ax == 1) {
+    sweep_t<3, 1>(s, g, dir, src, dst, code, c);
+  } else {
+    sweep_t<3, 2>(s, g, dir, src, dst, code, c);
+  }
+}
+
 int check_grid(int dim, const int32_t* res) {
   MG_REQUIRE(dim == 2 || dim == 3, "dim must be 2 or 3");
   MG_REQUIRE(res != nullptr, "res is NULL");
@@ -293,20 +552,28 @@ extern "C" int mgpcg_redistance(void* stream, int dim, const int32_t* res, doubl
   c.dx2 = (float)(dx * dx);
   c.half = (float)(1.0 / 2.0);
   c.third = (float)(1.0 / 3.0);
-  hipLaunchKernelGGL(k_target_surface, dim3(nblk(n)), dim3(LB), 0, s, g, (const float*)phi,
-                     (float)dx, phi_temp, fixed);
+  if (dim == 3)
+    hipLaunchKernelGGL((k_target_surface<3>), dim3(nblk(n)), dim3(LB), 0, s, g,
+                       (const float*)phi, (float)dx, phi_temp, fixed);
+  else
+    hipLaunchKernelGGL((k_target_surface<2>), dim3(nblk(n)), dim3(LB), 0, s, g,
+                       (const float*)phi, (float)dx, phi_temp, fixed);
+  // each sweep reads one work array and writes the other; the last one writes
+  // phi, which nothing reads after target_surface
+  const float* src = phi_temp;
+  float* dst = snap;
   for (int rep = 0; rep < repeat_times; ++rep) {
     for (int ax = dim - 1; ax >= 0; --ax) {
       for (int dir = 1; dir >= -1; dir -= 2) {
-        hipLaunchKernelGGL(k_copy, dim3(nblk(n)), dim3(LB), 0, s, n, (const float*)phi_temp,
-                           snap);
-        hipLaunchKernelGGL(k_sweep, dim3(nblk(n / g.n[ax])), dim3(LB), 0, s, g, ax, dir,
-                           (const float*)phi, (const float*)snap, phi_temp,
-                           (const int8_t*)fixed, c);
+        float* out = rep == repeat_times - 1 && ax == 0 && dir == -1 ? phi : dst;
+        sweep(s, g, ax, dir, src, out, (const int8_t*)fixed, c);
+        dst = const_cast<float*>(src);
+        src = out;
       }
     }
   }
-  hipLaunchKernelGGL(k_copy, dim3(nblk(n)), dim3(LB), 0, s, n, (const float*)phi_temp, phi);
+  if (repeat_times == 0)
+    hipLaunchKernelGGL(k_copy, dim3(nblk(n)), dim3(LB), 0, s, n, (const float*)phi_temp, phi);
   MG_HIP(hipGetLastError());
   return 0;
 }

@@ -104,3 +104,25 @@ def test_redistance_matches_oracle(dev, res, repeat):
     ls.redistance()
     ref = OL.redistance(phi, dx, repeat)
     assert np.array_equal(ls.phi.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("res", [(2, 2), (63, 2), (64, 15), (65, 16), (7, 17), (9, 33),
+                                 (2, 2, 2), (7, 9, 16), (8, 8, 17), (5, 13, 31), (17, 3, 33),
+                                 (3, 65, 15)], ids=lambda r: "x".join(map(str, r)))
+def test_redistance_at_tile_edges(dev, res):
+    """Lines and chunks that end inside, at and just past a tile of the sweep
+    kernels (64 lines, 16 steps along the contiguous axis, 8 on the others),
+    with infinities and repeated zeros in the level set: bit for bit."""
+    from mgpcg_amd.level_set import FastSweepingLevelSet
+
+    rng = np.random.default_rng(list(res))
+    phi = rng.normal(size=res).astype(np.float32)
+    phi[rng.uniform(size=res) < 0.7] = 1.5
+    phi[rng.uniform(size=res) < 0.05] = 0.0
+    phi[rng.uniform(size=res) < 0.03] = np.inf
+    dx = 0.37
+    ls = FastSweepingLevelSet(len(res), res, dx, phi=_t(phi, dev), device=dev)
+    ls.redistance()
+    with np.errstate(all="ignore"):
+        ref = OL.redistance(phi, dx, 2)
+    assert np.array_equal(ls.phi.cpu().numpy(), ref, equal_nan=True)
