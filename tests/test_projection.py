@@ -162,3 +162,32 @@ def test_extrap_velocity_closed_form():
         reach[k] = slice(7, 18)
         assert np.all(out[k][tuple(reach)] == np.float32(c))  # three layers out
         assert np.all(out[k][:5, :] == 9.0) and np.all(out[k][:, :5] == 9.0)  # beyond reach
+
+
+@pytest.mark.parametrize("res", [(2, 2), (3, 31), (5, 32), (4, 33), (9, 63), (2, 2, 2),
+                                 (2, 3, 31), (3, 4, 32), (5, 2, 65), (6, 7, 20)],
+                         ids=lambda r: "x".join(map(str, r)))
+@pytest.mark.parametrize("p_fluid", [0.0, 0.02, 1.0])
+def test_extrap_velocity_at_flag_words(dev, res, p_fluid):
+    """Rows that end inside, at and just past a 32-bit word of face flags and a
+    wave's 64 faces; no fluid at all, a few cells and all of them; a few faces
+    of infinite and NaN velocity: bit for bit."""
+    from mgpcg_amd import projection
+    from oracle import levelset as OL
+
+    rng = np.random.default_rng([*res, int(100 * p_fluid)])
+    ct = np.where(rng.uniform(size=res) < p_fluid, 0, 1).astype(np.int8)
+    if p_fluid == 0.02:
+        ct.flat[rng.integers(0, ct.size)] = 0
+    vel = []
+    for k in range(len(res)):
+        u = rng.normal(size=[n + (a == k) for a, n in enumerate(res)]).astype(np.float32)
+        u[rng.uniform(size=u.shape) < 0.02] = np.inf
+        u[rng.uniform(size=u.shape) < 0.02] = np.nan
+        vel.append(u)
+    for iters in (1, 4):
+        ref = OL.extrap_velocity(ct, [u.copy() for u in vel], iters)
+        v = [_t(u, dev) for u in vel]
+        projection.extrap_velocity(v, _t(ct, dev), iters)
+        for a, b in zip(v, ref):
+            assert np.array_equal(a.cpu().numpy(), b, equal_nan=True)
