@@ -60,6 +60,12 @@ __device__ __forceinline__ void stgi(T* base, int i, T v) {
 #define MG_READLANE(v, l) __builtin_amdgcn_readlane((v), (l))
 #endif
 
+// A 32-bit value that is the same in every lane, as a scalar (the compiler
+// then addresses through scalar registers).
+#ifndef MG_UNIFORM
+#define MG_UNIFORM(v) __builtin_amdgcn_readfirstlane(v)
+#endif
+
 #ifndef MG_KEEP
 #define MG_KEEP(x) asm volatile("" ::"v"(x))
 #define MG_KEEP4(a, b, c, d) asm volatile("" ::"v"(a), "v"(b), "v"(c), "v"(d))

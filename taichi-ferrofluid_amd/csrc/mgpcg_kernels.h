@@ -178,6 +178,7 @@ struct Stage {
   const Item* items;
   int nitems;
   int nblocks;  // total virtual blocks
+  Item one;     // items[0]: with one system, no load stands before its descriptor's
   // measurement only: when non-NULL, a level-0 smooth(0) launch adds the
   // level-0 cells of every system it sweeps (done systems are skipped) to
   // swept[0] and their FLUID cells to swept[1], and its span on the device's
@@ -473,12 +474,16 @@ struct ItemCache {
 };
 __device__ __forceinline__ bool item_at(const Stage& S, int vb, ItemCache& c) {
   if (vb >= c.begin && vb < c.end) return false;
-  const int ii = find_item(S.items, S.nitems, vb);
-  const Item it = S.items[ii];
-  c.desc = it.desc;
-  c.block0 = it.block0;
-  c.begin = it.block0;
-  c.end = ii + 1 < S.nitems ? S.items[ii + 1].block0 : S.nblocks;
+  Item it = S.one;
+  int end = S.nblocks;
+  if (S.nitems > 1) {
+    const int ii = find_item(S.items, S.nitems, vb);
+    it = S.items[ii];
+    if (ii + 1 < S.nitems) end = S.items[ii + 1].block0;
+  }
+  c.desc = MG_UNIFORM(it.desc);
+  c.block0 = c.begin = MG_UNIFORM(it.block0);
+  c.end = MG_UNIFORM(end);
   return true;
 }
 
@@ -1344,6 +1349,405 @@ __global__ void __launch_bounds__(BLOCK) k_restrict_gather(const LevelDesc<T>* _
       for (int o = 0; o < (DIM == 3 ? 8 : 4); ++o) sum = sum + v[o];
       stgi(cc ? D.C.r[1] : D.C.r[0], tc, sum);
     }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// fused V-cycle legs: a level's whole pre-smoothing with the restriction, or
+// its prolongation with the whole post-smoothing, in one launch
+// ---------------------------------------------------------------------------
+// A launch of a half-sweep on a level of a few thousand to a few hundred
+// thousand cells takes 4-5 us whatever it does: each workgroup waits for its
+// descriptor, its work order and then its operands, and the level has ten such
+// launches per V-cycle.  Here a workgroup takes a block of the level
+// with the TILE_HALO layers around it, keeps every cell's right-hand side,
+// diagonal and couplings in registers and z in LDS, and runs all the leg's
+// half-sweeps on it, each valid one layer further in; the layers are computed
+// by every workgroup that needs them, so no workgroup waits for another.  The
+// values are the half-sweep kernels', operation for operation.
+//
+// 3D: 8^3 cells in a 16^3 block (4.1 slot updates per useful one), 1024 lanes
+// of two slots per colour; 2D: 24^2 in 32^2, 512 lanes of one slot.
+// A leg takes 7.6-8.4 us on 32^3 cells (64 blocks) and 14 us on 64^3 (512, 30%
+// of them wet) where its launches took 27 and 30 us (before) and 19 and 22 us
+// (after); 6 us on a 128^2 level 0 for 21 us.  What is left is the launch, the
+// two dependent reads before the first operand, and VALU issue: 38 instructions
+// per slot update, the exact division 10 of them.  80 VGPRs leave one 3D
+// workgroup per CU; asked for two (64 VGPRs, 14 spilled) a 128^3 solve went
+// from 4.32 to 4.55 ms.  Whole solves: 128^2 1055 -> 857 us, 128^3 5.33 ->
+// 4.35 ms, 256^3 20.5 -> 19.2 ms.
+constexpr int TILE_HALO = 4;      // deepest dependency chain of a leg that fits
+constexpr int TILE_MAX_NU = 2;    // smoothing steps: 2 * nu half-sweeps <= TILE_HALO
+template <int DIM>
+struct TileShape {
+  static constexpr int S = DIM == 3 ? 16 : 32;      // edge of the block with its layers
+  static constexpr int CORE = S - 2 * TILE_HALO;    // edge of the part that is stored
+  static constexpr int CELLS = DIM == 3 ? S * S * S : S * S;
+  static constexpr int NT = DIM == 3 ? 1024 : 512;
+  static constexpr int NS = CELLS / 2 / NT;         // slots per lane and colour
+  static constexpr int CC = CORE / 2;               // coarse cells along the core
+  static constexpr int COARSE = DIM == 3 ? CC * CC * CC : CC * CC;
+  // LDS stride of original axis a
+  __host__ __device__ static constexpr int stride(int a) {
+    return DIM == 3 ? (a == 0 ? S * S : (a == 1 ? S : 1)) : (a == 0 ? S : 1);
+  }
+};
+template <int DIM>
+__host__ __device__ inline int tile_count(const Geo& g) {
+  constexpr int C = TileShape<DIM>::CORE;
+  return (DIM == 3 ? (g.n0 + C - 1) / C : 1) * ((g.n1 + C - 1) / C) * ((g.n2 + C - 1) / C);
+}
+
+// One slot of a block: its place, how many layers lie outside it, and its row
+// of the operator.
+template <typename T, int DIM>
+struct TileCell {
+  int t;      // slot in the level's colour array (0, a ghost slot, outside the level)
+  int loc;    // cell in the LDS block
+  int depth;  // layers of the block outside the cell
+  bool inside, fluid;
+  T r, ad, al[DIM], ah[DIM];
+};
+
+// place of slot u of colour c of the block whose first cell is (oi, oj, ok)
+// (even coordinates, so a cell's colour is the parity of its block coordinates)
+template <typename T, int DIM>
+__device__ __forceinline__ void tile_place(const Geo& g, int oi, int oj, int ok, int u, int c,
+                                           TileCell<T, DIM>& v) {
+  using Ts = TileShape<DIM>;
+  constexpr int RS = Ts::S / 2;
+  const int row = u / RS, m = u % RS;
+  const int a = DIM == 3 ? row / Ts::S : 0, b = row % Ts::S;
+  const int e = 2 * m + ((a + b + c) & 1);
+  v.loc = row * Ts::S + e;
+  const int far = Ts::S - 1;
+  v.depth = min(min(b, far - b), min(e, far - e));
+  if (DIM == 3) v.depth = min(v.depth, min(a, far - a));
+  const int i = DIM == 3 ? oi + a : 0, j = oj + b, k = ok + e;
+  v.inside = i >= 0 && i < g.n0 && j >= 0 && j < g.n1 && k >= 0 && k < g.n2;
+  v.t = v.inside ? slot_of(g, i, j, k) : 0;
+}
+
+// Right-hand side, diagonal and flag word of every slot of a lane (slots
+// outside the level read a ghost slot's zeros).  Issued before the system's
+// state and the level's coupling summary are looked at: those loads and these
+// are one wait, not two.
+template <typename T, int DIM>
+__device__ __forceinline__ void tile_rows(const LevelPtrs<T>& P, TileCell<T, DIM>* v,
+                                          uint32_t* f) {
+#pragma unroll
+  for (int u = 0; u < 2 * TileShape<DIM>::NS; ++u) {
+    v[u].r = ldgi(P.r[u & 1], v[u].t);
+    v[u].ad = ldgi(P.Adiag[u & 1], v[u].t);
+    f[u] = ldgi(P.nb[u & 1], v[u].t);
+  }
+}
+template <typename T, int DIM>
+__device__ __forceinline__ void tile_keep(TileCell<T, DIM>* v, uint32_t* f) {
+#pragma unroll
+  for (int u = 0; u < 2 * TileShape<DIM>::NS; ++u) {
+    MG_KEEP(v[u].r);
+    MG_KEEP(v[u].ad);
+    MG_KEEP(f[u]);
+  }
+}
+
+// The slots' couplings and FLUID marks: from the flag words on a level with
+// uniform couplings, else the stored couplings and cell types.
+template <typename T, int DIM>
+__device__ __forceinline__ void tile_couplings(const Geo& g, const LevelPtrs<T>& P,
+                                               const Coupling<T>& kc, const uint32_t* f,
+                                               TileCell<T, DIM>* v) {
+  constexpr int N = 2 * TileShape<DIM>::NS;
+  if (kc.uniform) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      v[u].fluid = v[u].inside && ((f[u] >> NB_FL) & 1u) != 0u;
+#pragma unroll
+      for (int a = 0; a < DIM; ++a) {
+        v[u].al[a] = ((f[u] >> (NB_DN + a)) & 1u) ? kc.coef : (T)0;
+        v[u].ah[a] = ((f[u] >> a) & 1u) ? kc.coef : (T)0;
+      }
+    }
+    return;
+  }
+  int gt[N];
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const int c = u & 1;
+    gt[u] = ldgi(P.gt[c], v[u].t);
+    const Nbr<DIM> n = neighbours_clamped<DIM>(g, v[u].t, row_q(g, v[u].t, c));
+#pragma unroll
+    for (int a = 0; a < DIM; ++a) {
+      v[u].al[a] = ldgi(P.Ax[a][c ^ 1], n.lo[a]);
+      v[u].ah[a] = ldgi(P.Ax[a][c], v[u].t);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    MG_KEEP(gt[u]);
+#pragma unroll
+    for (int a = 0; a < DIM; ++a) {
+      MG_KEEP(v[u].al[a]);
+      MG_KEEP(v[u].ah[a]);
+    }
+    v[u].fluid = v[u].inside && gt[u] == MG_FLUID;
+  }
+}
+
+template <typename T, int DIM>
+__device__ __forceinline__ T tile_nsum(const T* z, const TileCell<T, DIM>& v) {
+  T zl[DIM], zh[DIM];
+#pragma unroll
+  for (int a = 0; a < DIM; ++a) {
+    zl[a] = z[v.loc - TileShape<DIM>::stride(a)];
+    zh[a] = z[v.loc + TileShape<DIM>::stride(a)];
+  }
+  return nsum_vals<T, DIM>(v.al, v.ah, zl, zh);
+}
+
+// first cell of the block with its layers: block `tile` of the level
+template <int DIM>
+__device__ __forceinline__ void tile_origin(const Geo& g, int tile, int& oi, int& oj, int& ok) {
+  constexpr int C = TileShape<DIM>::CORE;
+  const int nk = (g.n2 + C - 1) / C, nj = (g.n1 + C - 1) / C;
+  const int row = tile / nk;
+  ok = (tile - row * nk) * C - TILE_HALO;
+  const int pl = DIM == 3 ? row / nj : 0;
+  oj = (row - pl * nj) * C - TILE_HALO;
+  oi = DIM == 3 ? pl * C - TILE_HALO : 0;
+}
+
+// z.fill(0), nu smoothing steps (mgpcg.py:126-131), restrict(l) (:111-118):
+// colour 0 of z goes to the level's scratch res[0] (the other leg reads it
+// while its workgroups write z; colour 1 is rewritten there before it is
+// read), the restricted residual to the coarser level's r.
+template <typename T, int DIM>
+__global__ void __launch_bounds__(TileShape<DIM>::NT) k_tile_pre(
+    const LevelDesc<T>* __restrict__ descs, Stage S, int nu) {
+  using Ts = TileShape<DIM>;
+  constexpr int NS = Ts::NS;
+  __shared__ T z[Ts::CELLS];
+  __shared__ T res[Ts::CELLS];
+  __shared__ int any;
+  ItemCache ic;
+  int done = 1;
+  Coupling<T> kc{false, (T)0};
+  for (VBIter it = vb_begin(S.nblocks); it.vb < it.end; it.vb += it.step) {
+    const bool fresh = item_at(S, it.vb, ic);
+    const LevelDesc<T>& D = descs[ic.desc];
+    int oi, oj, ok;
+    tile_origin<DIM>(D.g, it.vb - ic.block0, oi, oj, ok);
+    __syncthreads();  // the previous block's LDS reads are done
+    if (threadIdx.x == 0) any = 0;
+    TileCell<T, DIM> v[2 * NS];  // [slot][colour]
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        tile_place<T, DIM>(D.g, oi, oj, ok, s * Ts::NT + (int)threadIdx.x, c, v[2 * s + c]);
+    uint32_t f[2 * NS];
+    tile_rows<T, DIM>(D.P, v, f);
+    if (fresh) {
+      done = ldg(&D.st->done);
+      kc = coupling_g(D.P);
+    }
+    tile_keep<T, DIM>(v, f);
+    if (done) continue;
+    tile_couplings<T, DIM>(D.g, D.P, kc, f, v);
+    __syncthreads();
+    T own[2 * NS], rs[NS];
+    bool mine = false;  // a FLUID cell of the core
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      own[2 * s] = v[2 * s].fluid ? v[2 * s].r / v[2 * s].ad : (T)0;
+      own[2 * s + 1] = (T)0;
+      rs[s] = (T)0;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        z[v[2 * s + c].loc] = own[2 * s + c];
+        mine = mine || (v[2 * s + c].fluid && v[2 * s + c].depth >= TILE_HALO);
+      }
+    }
+    if (mine) any = 1;
+    __syncthreads();
+    const bool wet = any != 0;
+    if (wet) {
+      for (int h = 1; h < 2 * nu; ++h) {  // half-sweeps 1, 0, 1, ...
+        if (h & 1) {
+          const bool last = h == 2 * nu - 1;
+#pragma unroll
+          for (int s = 0; s < NS; ++s) {
+            const TileCell<T, DIM>& x = v[2 * s + 1];
+            if (!x.fluid || x.depth < h) continue;
+            const T sm = tile_nsum<T, DIM>(z, x);
+            const T num = x.r - sm;
+            const T zn = num / x.ad;
+            own[2 * s + 1] = zn;
+            z[x.loc] = zn;
+            if (last) {
+              T Az = x.ad * zn;
+              Az = Az + sm;
+              rs[s] = x.r - Az;
+            }
+          }
+        } else {
+#pragma unroll
+          for (int s = 0; s < NS; ++s) {
+            const TileCell<T, DIM>& x = v[2 * s];
+            if (!x.fluid || x.depth < h) continue;
+            const T sm = tile_nsum<T, DIM>(z, x);
+            const T num = x.r - sm;
+            own[2 * s] = num / x.ad;
+            z[x.loc] = own[2 * s];
+          }
+        }
+        __syncthreads();
+      }
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        const TileCell<T, DIM>& x1 = v[2 * s + 1];
+        if (x1.depth >= TILE_HALO) res[x1.loc] = rs[s];
+        const TileCell<T, DIM>& x = v[2 * s];
+        if (x.depth < TILE_HALO) continue;
+        T rr = (T)0;
+        if (x.fluid) {
+          const T ns = tile_nsum<T, DIM>(z, x);
+          T Az = x.ad * own[2 * s];
+          Az = Az + ns;
+          rr = x.r - Az;
+          stgi(D.P.res[0], x.t, own[2 * s]);
+        }
+        res[x.loc] = rr;
+      }
+      __syncthreads();
+    }
+    // every coarse cell sums its children in lexicographic order
+    if ((int)threadIdx.x < Ts::COARSE) {
+      const int w = threadIdx.x;
+      const int a = DIM == 3 ? w / (Ts::CC * Ts::CC) : 0;
+      const int b = (w / Ts::CC) % Ts::CC, e = w % Ts::CC;
+      const int i = DIM == 3 ? ((oi + TILE_HALO) >> 1) + a : 0;
+      const int j = ((oj + TILE_HALO) >> 1) + b, k = ((ok + TILE_HALO) >> 1) + e;
+      if (i < D.gc.n0 && j < D.gc.n1 && k < D.gc.n2) {
+        T sum = (T)0;
+        if (wet) {
+          const int base = (DIM == 3 ? (2 * a + TILE_HALO) * Ts::S * Ts::S : 0) +
+                           (2 * b + TILE_HALO) * Ts::S + 2 * e + TILE_HALO;
+#pragma unroll
+          for (int o0 = 0; o0 < (DIM == 3 ? 2 : 1); ++o0)
+#pragma unroll
+            for (int o1 = 0; o1 < 2; ++o1)
+#pragma unroll
+              for (int o2 = 0; o2 < 2; ++o2)
+                sum = sum + res[base + o0 * Ts::S * Ts::S + o1 * Ts::S + o2];
+        }
+        stgi(colour_of(i, j, k) ? D.C.r[1] : D.C.r[0], slot_of(D.gc, i, j, k), sum);
+      }
+    }
+  }
+}
+
+// prolongate(l) (mgpcg.py:120-123) and nu smoothing steps (:143-147).  L0:
+// without the last smooth(0, 0), which the kernel that also forms z.r does,
+// and with colour 1 only stored.
+template <typename T, int DIM, bool L0>
+__global__ void __launch_bounds__(TileShape<DIM>::NT) k_tile_post(
+    const LevelDesc<T>* __restrict__ descs, Stage S, int nu) {
+  using Ts = TileShape<DIM>;
+  constexpr int NS = Ts::NS;
+  __shared__ T z[Ts::CELLS];
+  __shared__ int any;
+  ItemCache ic;
+  int done = 1;
+  Coupling<T> kc{false, (T)0};
+  for (VBIter it = vb_begin(S.nblocks); it.vb < it.end; it.vb += it.step) {
+    const bool fresh = item_at(S, it.vb, ic);
+    const LevelDesc<T>& D = descs[ic.desc];
+    int oi, oj, ok;
+    tile_origin<DIM>(D.g, it.vb - ic.block0, oi, oj, ok);
+    __syncthreads();  // the previous block's LDS reads are done
+    if (threadIdx.x == 0) any = 0;
+    TileCell<T, DIM> v[2 * NS];  // [slot][colour]
+    T zv[NS], pv[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        tile_place<T, DIM>(D.g, oi, oj, ok, s * Ts::NT + (int)threadIdx.x, c, v[2 * s + c]);
+      const TileCell<T, DIM>& x = v[2 * s];
+      // the parent's z: outside the level a ghost slot's, which is 0
+      constexpr int SS = Ts::S;
+      const int i = DIM == 3 ? oi + x.loc / (SS * SS) : 0;
+      const int j = oj + (x.loc / SS) % SS, k = ok + x.loc % SS;
+      const int pi = i >> 1, pj = j >> 1, pk = k >> 1;
+      const int ps = x.inside ? slot_of(D.gc, pi, pj, pk) : 0;
+      zv[s] = ldgi(D.P.res[0], x.t);
+      pv[s] = ldgi(colour_of(pi, pj, pk) ? D.C.z[1] : D.C.z[0], ps);
+    }
+    uint32_t f[2 * NS];
+    tile_rows<T, DIM>(D.P, v, f);
+    if (fresh) {
+      done = ldg(&D.st->done);
+      kc = coupling_g(D.P);
+    }
+    tile_keep<T, DIM>(v, f);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      MG_KEEP(zv[s]);
+      MG_KEEP(pv[s]);
+    }
+    if (done) continue;
+    tile_couplings<T, DIM>(D.g, D.P, kc, f, v);
+    __syncthreads();
+    T own[2 * NS];
+    bool mine = false;  // a FLUID cell of the core
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const TileCell<T, DIM>& x = v[2 * s];
+      z[x.loc] = x.inside ? zv[s] + pv[s] : (T)0;
+      z[v[2 * s + 1].loc] = (T)0;
+      own[2 * s] = own[2 * s + 1] = (T)0;
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        mine = mine || (v[2 * s + c].fluid && v[2 * s + c].depth >= TILE_HALO);
+    }
+    if (mine) any = 1;
+    __syncthreads();
+    if (any == 0) continue;
+    for (int h = 1; h <= 2 * nu - (L0 ? 1 : 0); ++h) {  // half-sweeps 1, 0, 1, ...
+      if (h & 1) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          const TileCell<T, DIM>& x = v[2 * s + 1];
+          if (!x.fluid || x.depth < h) continue;
+          const T sm = tile_nsum<T, DIM>(z, x);
+          const T num = x.r - sm;
+          own[2 * s + 1] = num / x.ad;
+          z[x.loc] = own[2 * s + 1];
+        }
+      } else {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          const TileCell<T, DIM>& x = v[2 * s];
+          if (x.depth < h) continue;
+          if (x.fluid) {
+            const T sm = tile_nsum<T, DIM>(z, x);
+            const T num = x.r - sm;
+            own[2 * s] = num / x.ad;
+          }
+          z[x.loc] = own[2 * s];  // off FLUID: z without the prolongation, 0
+        }
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+      for (int c = L0 ? 1 : 0; c < 2; ++c) {
+        const TileCell<T, DIM>& x = v[2 * s + c];
+        if (x.fluid && x.depth >= TILE_HALO) stgi(D.P.z[c], x.t, own[2 * s + c]);
+      }
   }
 }
 

@@ -68,6 +68,7 @@ int g_coarse_lds = 1;    // coarse kernel works on an LDS image of its levels wh
 // pass + child gather (both coalesced)
 int g_restrict_mode = 2;
 int g_restrict_coarse = -1;  // restriction kernels on levels >= 1 (-1: g_restrict_mode)
+int g_tile_max = 768;     // most 3D blocks a launch of the fused V-cycle legs takes (0: never)
 int g_probe_every = 4;    // the launch probe times one eligible launch in this many
 int g_server_depth = 2;   // server iterations queued on the device ahead of the host
 int g_server_streams = 2; // engines (streams) a server spreads its members over
@@ -244,6 +245,7 @@ struct Engine {
   std::vector<Item> items;
   struct StageRef {
     int off = 0, n = 0, nblocks = 0;
+    Item one{0, 0};  // the first item
     int fine_nblocks = 0;  // one-item restriction stages: the fine level's slot blocks
   };
   StageRef st_init, st_cg, fin_init, fin_cg, fin_all, st_dot_fused, st_dot_plain, st_coarse,
@@ -252,6 +254,7 @@ struct Engine {
   int restrict_mode = 0;    // restriction stages of level 0 are laid out for this mode
   int restrict_mode_c = 0;  // ... and those of the levels below it for this one
   std::vector<StageRef> st_slot, st_restrict, st_bottom;  // per level
+  std::vector<StageRef> st_tile;  // per level: the fused legs' blocks
   // the half-sweep stages: virtual blocks of BLOCK * SLOT_LANES slots
   std::vector<StageRef> st_sweep, st_bottom_sweep;
   int n_items_cap = 0;
@@ -523,6 +526,7 @@ int engine_configure(Engine* e, const mgpcg_solver* s) {
   e->level_sz = level_desc_size(e->precision);
   e->sys_sz = sys_desc_size(e->precision);
   e->st_slot.assign(e->L, {});
+  e->st_tile.assign(e->L, {});
   e->st_sweep.assign(e->L, {});
   e->st_bottom_sweep.assign(1, {});
   e->st_restrict.assign(e->L, {});
@@ -618,6 +622,7 @@ int engine_build_items(Engine* e) {
       b0 += blocks(M);
     }
     ref.n = (int)it.size() - ref.off;
+    ref.one = ref.n > 0 ? it[ref.off] : Item{0, 0};
     ref.nblocks = b0;
   };
   const int L = e->L;
@@ -645,6 +650,13 @@ int engine_build_items(Engine* e) {
               [l, L](int m) { return m * L + l; });
     add_stage(e->st_sweep[l], [l](const Member& M) { return l < M.s->coarse_from; },
               [l](const Member& M) { return nsweep(M.s->geo[l].size); },
+              [l, L](int m) { return m * L + l; });
+    add_stage(e->st_tile[l],
+              [l, L](const Member& M) { return l < M.s->coarse_from && l + 1 < L; },
+              [l](const Member& M) {
+                const Geo& g = M.s->geo[l];
+                return g.dim == 3 ? tile_count<3>(g) : tile_count<2>(g);
+              },
               [l, L](int m) { return m * L + l; });
     add_stage(e->st_restrict[l],
               [l, L](const Member& M) { return l < M.s->coarse_from && l + 1 < L; },
@@ -739,6 +751,7 @@ inline Stage stage_of(const Engine* e, const Engine::StageRef& r) {
   s.items = e->d_items + r.off;
   s.nitems = r.n;
   s.nblocks = r.nblocks;
+  s.one = r.one;
   s.swept = nullptr;
   s.t0 = nullptr;
   s.t1 = nullptr;
@@ -805,12 +818,33 @@ struct Sched {
                        (const Item*)(e->d_items + r.off), r.n, out);
   }
 
+  // Whether level l runs as the two fused legs (an option that selects other
+  // half-sweep or restriction kernels keeps those).  A 3D block costs a CU
+  // about 5 us a leg, so the legs' time grows with the blocks per CU, while
+  // the half-sweeps' ten launches cost 4-5 us each until their traffic counts.
+  // Measured, half-sweeps against legs, whole solves: level 1 of 72x48x88
+  // (594 blocks) 4.71 -> 4.46 ms; of 88x80x72, all FLUID (990) 54.9 -> 60.2 ms;
+  // level 0 of 96x112x88 (1848) 2.65 -> 3.48 ms.  A 2D block has a quarter of
+  // the cells and little overlap: 1024^2 (1849 blocks) 3.75 -> 3.37 ms.
+  static bool tiled(const Engine* e, int l) {
+    const long n = e->st_tile[l].nblocks, most = (DIM == 3 ? 1l : 4l) * g_tile_max;
+    return n > 0 && n <= most && e->nu >= 1 && e->nu <= TILE_MAX_NU &&
+           g_fuse_first == 0 && g_fuse_prolong && restrict_mode_of(e, l) == 2 &&
+           !(l == 0 && e->probe_on);  // the probe times level 0's half-sweeps
+  }
+
   // v_cycle (mgpcg.py:125-148) for every member.  first0: level 0's first
   // half-sweep from z = 0 was done by the kernel that wrote r (k_cg_init,
   // k_cg_xr, k_true_residual).
   static void vcycle(Engine* e, bool first0 = false) {
     const int L = e->L, nu = e->nu;
     for (int l = 0; l + 1 < L; ++l) {
+      if (tiled(e, l)) {
+        const Engine::StageRef& t = e->st_tile[l];
+        hipLaunchKernelGGL((k_tile_pre<T, DIM>), dim3(grid_of(t)), dim3(TileShape<DIM>::NT), 0,
+                           e->stream, levels(e), stage_of(e, t), nu);
+        continue;
+      }
       const Engine::StageRef& S = e->st_slot[l];
       const Engine::StageRef& W = e->st_sweep[l];
       // the last pre-smoothing smooth(l, 1) also forms the colour-1 residual
@@ -871,6 +905,18 @@ struct Sched {
                            e->st_coarse.n, nu, e->bottom);
     }
     for (int l = L - 2; l >= 0; --l) {
+      if (tiled(e, l)) {
+        const Engine::StageRef& t = e->st_tile[l];
+        if (l == 0)
+          hipLaunchKernelGGL((k_tile_post<T, DIM, true>), dim3(grid_of(t)),
+                             dim3(TileShape<DIM>::NT), 0, e->stream, levels(e), stage_of(e, t),
+                             nu);
+        else
+          hipLaunchKernelGGL((k_tile_post<T, DIM, false>), dim3(grid_of(t)),
+                             dim3(TileShape<DIM>::NT), 0, e->stream, levels(e), stage_of(e, t),
+                             nu);
+        continue;
+      }
       const Engine::StageRef& S = e->st_slot[l];
       const Engine::StageRef& W = e->st_sweep[l];
       if (nu > 0) {
@@ -1470,6 +1516,10 @@ extern "C" int mgpcg_set_option(mgpcg_solver_t* s, int option, int value) {
       MG_REQUIRE(value >= -1 && value <= 2, "coarse restriction mode must be -1, 0, 1 or 2");
       g_restrict_coarse = value;
       return 0;
+    case MGPCG_OPT_TILE_MAX:
+      MG_REQUIRE(value >= 0, "block limit must be >= 0");
+      g_tile_max = value;
+      return 0;
     case MGPCG_OPT_PROBE_EVERY:
       MG_REQUIRE(value >= 1, "probe period must be >= 1");
       g_probe_every = value;
@@ -1507,6 +1557,7 @@ extern "C" int mgpcg_get_option(const mgpcg_solver_t* s, int option, int* value)
     case MGPCG_OPT_COARSE_LDS: *value = g_coarse_lds; return 0;
     case MGPCG_OPT_RESTRICT_ROWS: *value = g_restrict_mode; return 0;
     case MGPCG_OPT_RESTRICT_COARSE: *value = g_restrict_coarse; return 0;
+    case MGPCG_OPT_TILE_MAX: *value = g_tile_max; return 0;
     case MGPCG_OPT_PROBE_EVERY: *value = g_probe_every; return 0;
     case MGPCG_OPT_SERVER_DEPTH: *value = g_server_depth; return 0;
     case MGPCG_OPT_SERVER_STREAMS: *value = g_server_streams; return 0;
@@ -1782,6 +1833,7 @@ struct RefPath {
     auto lvl = [&](int l, bool coarse) {
       Engine::StageRef r;
       r.off = l;
+      r.one = it[l];
       r.n = 1;
       r.nblocks = coarse ? restrict_blocks(e, s->geo[l + 1]) : nblk(s->geo[l].size);
       return r;
@@ -1789,6 +1841,7 @@ struct RefPath {
     auto sweep = [&](int l) {  // a half-sweep stage of level l
       Engine::StageRef r;
       r.off = l;
+      r.one = it[l];
       r.n = 1;
       r.nblocks = nsweep(s->geo[l].size);
       return r;
@@ -2003,6 +2056,7 @@ int prepare_op(Engine* e, const mgpcg_solver* s, int op, int level, Engine::Stag
   MG_HIP(hipStreamSynchronize(e->stream));
   MG_HIP(hipMemcpy(e->d_items, &it, sizeof(Item), hipMemcpyHostToDevice));
   r->off = 0;
+  r->one = it;
   r->n = 1;
   r->nblocks = nb;
   e->dirty = true;  // the item table no longer matches the member set

@@ -20,7 +20,7 @@ FIELD_R, FIELD_Z, FIELD_P, FIELD_AP, FIELD_X, FIELD_P_NEXT = 0, 1, 2, 3, 4, 5
 (OPT_COARSE_MAX_SLOTS, OPT_MAX_GRID, OPT_FUSE_FIRST, OPT_FUSE_PROLONG, OPT_FUSE_P,
  OPT_COMPACT, OPT_COARSE_LDS, OPT_RESTRICT_ROWS, OPT_PROBE_EVERY,
  OPT_SERVER_DEPTH, OPT_SERVER_STREAMS, OPT_GRAPH,
- OPT_RESTRICT_COARSE) = 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15
+ OPT_RESTRICT_COARSE, OPT_TILE_MAX) = 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16
 
 _P = ctypes.c_void_p
 _I = ctypes.c_int
