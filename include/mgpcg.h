@@ -79,9 +79,9 @@ int mgpcg_set_stream(mgpcg_solver_t* solver, void* stream);
 #define MGPCG_OPT_COMPACT 8       /* 1: levels whose nonzero off-diagonals are all one value
                                      read per-cell coupling flags instead of Ax (default 1);
                                      applies to systems solved or submitted afterwards */
-#define MGPCG_OPT_COARSE_LDS 9    /* 1: the coarse-level kernel runs on a copy of its levels'
-                                     cell types, flags, Adiag, r and z in LDS (160 KB) when
-                                     they fit (FP32 hierarchies; default 1) */
+#define MGPCG_OPT_COARSE_LDS 9    /* 1: the coarse-level kernel keeps its levels' z and
+                                     residuals in LDS (160 KB) and their operators in
+                                     registers when they fit (FP32 hierarchies; default 1) */
 #define MGPCG_OPT_RESTRICT_ROWS 10 /* restriction kernels: 2 a residual pass into scratch
                                       then a child gather (default), 1 tiled by coarse
                                       rows with the residuals in LDS (fine rows up to 512

@@ -62,8 +62,14 @@ __device__ __forceinline__ void stgi(T* base, int i, T v) {
 
 // A 32-bit value that is the same in every lane, as a scalar (the compiler
 // then addresses through scalar registers).
-#ifndef MG_UNIFORM
+#ifdef __HIP__
 #define MG_UNIFORM(v) __builtin_amdgcn_readfirstlane(v)
+// What is computed from x after this point is computed there (not hoisted out
+// of a loop and held in registers).
+#define MG_HERE(x) asm volatile("" : "+v"(x))
+#else
+#define MG_UNIFORM(v) (v)
+#define MG_HERE(x) ((void)(x))
 #endif
 
 #ifndef MG_KEEP

@@ -1904,429 +1904,419 @@ __device__ void coarse_bottom(const Geo& g, const LevelPtrs<T>& P, int bottom) {
 }
 
 // ---------------------------------------------------------------------------
-// The coarse V-cycle on its LDS image.  Every phase gives each lane up to
-// CZ_SLOTS slots and gathers the operands of all of them before computing any
-// (within a phase no slot reads a value the phase writes), then stores: a lane
-// keeps all its slots' LDS reads in flight together instead of one slot's
-// chain of reads at a time.  The arithmetic is the global-memory form's,
-// operation for operation (smooth_slot, restrict_slot, prolong_smooth1_slot).
+// the coarse kernel on LDS
 // ---------------------------------------------------------------------------
-constexpr int CZ_SLOTS = 3;
-// slots per lane of a phase that also gathers stored couplings (more
-// operands per slot: fewer slots keep them in registers)
-template <bool COMPACT>
+// One workgroup runs a system's coarse levels; a half-sweep of them is bound
+// by the vector instructions its one CU issues and, on the small levels, by
+// the chain of one slot's update between two barriers.  So a lane owns fixed
+// FLUID slots for the whole V-cycle: the FLUID slots of each level and colour
+// are listed once (ghost, AIR and SOLID slots cost nothing afterwards), and a
+// lane keeps each of its slots' right-hand side, couplings, diagonal and
+// reciprocal diagonal in registers; LDS holds z and the residuals.  Levels
+// with stored couplings (potential, surface tension) run the same phases.
+// The arithmetic is the global-memory form's, operation for operation.
+// Before, every phase decoded and re-read each slot of an LDS image of the
+// whole level: 32.8 -> 19.0 us a V-cycle at 128^3 (levels of 16^3 and 8^3
+// cells), 29.7 -> 19.7 us at 128^2, where a phase on the smallest level takes
+// 0.27 us; levels whose image did not fit ran from global memory (126 us for
+// a batch's 16 systems, 39 us now).  Solves: 128^3 4.32 -> 3.95 ms, 128^2
+// 857 -> 790 us, batch of 16 97 -> 75 ms.
+//
+// The first coarse level has at most CZ_MAX_SLOTS slots per colour; with its
+// ghost layers off, at most 3 cells per lane and colour in 3D
+// ((n0 + 2)(n1 + 2)(n2 + 3) / 2 <= 4096 gives n0 n1 n2 / 2 < 2830) and 4 in 2D.
+// The levels below have a fourth of its cells or fewer: one per lane.
+constexpr int CZ_MAX_SLOTS = 4096;
+template <int DIM>
 __host__ __device__ constexpr int cz_slots() {
-  return COMPACT ? CZ_SLOTS : 2;
+  return DIM == 3 ? 3 : 4;
+}
+constexpr int COARSE_LDS_BYTES = 160 * 1024 - 256;  // the rest: the lists' lengths
+constexpr int CZ_MAX_LEVELS = 16;
+__host__ __device__ constexpr int lds_align(int b) { return (b + 15) & ~15; }
+// a level's z, residual and right-hand side colour arrays and its FLUID lists
+__host__ __device__ constexpr int coarse_image_bytes(int size, int esz) {
+  return 6 * lds_align(size * esz) + 2 * lds_align(2 * size);
 }
 
-// operands of a half-sweep, or of a residual (own = the slot's z), at one
-// slot: on a level with uniform couplings (COMPACT) the flag word, else the
-// stored couplings (global memory, at clamped indices: a ghost slot's reads
-// stay in bounds and are discarded).  Only loads: the couplings are decoded
-// when the value is formed, so no read waits for another.
-template <typename T, int DIM, bool COMPACT>
-struct CzOps {
-  int gt;
-  uint32_t f;
-  T rv, ad, own;
-  T al[DIM], ah[DIM], zl[DIM], zh[DIM];
+template <typename T>
+struct CzLevel {
+  T *z[2], *res[2], *r[2];
+  uint16_t* list[2];
 };
-
-template <typename T, int DIM, bool COMPACT>
-__device__ __forceinline__ void cz_gather(const Geo& g, const LevelPtrs<T>& P, int c, int t,
-                                          bool own, CzOps<T, DIM, COMPACT>& v) {
-  const Nbr<DIM> n = neighbours_clamped<DIM>(g, t, row_q(g, t, c));
-  v.gt = P.gt[c][t];
-  v.rv = P.r[c][t];
-  v.ad = P.Adiag[c][t];
-  v.own = own ? P.z[c][t] : (T)0;
-  const T* zo = P.z[c ^ 1];
-#pragma unroll
-  for (int a = 0; a < DIM; ++a) {
-    v.zl[a] = zo[n.lo[a]];
-    v.zh[a] = zo[n.hi[a]];
-  }
-  if constexpr (COMPACT) {
-    v.f = P.nb[c][t];
-  } else {
-#pragma unroll
-    for (int a = 0; a < DIM; ++a) {
-      v.al[a] = P.Ax[a][c ^ 1][n.lo[a]];
-      v.ah[a] = P.Ax[a][c][t];
-    }
-  }
-}
-
-// the slot's couplings (decoded from the flag word on COMPACT levels)
-template <typename T, int DIM, bool COMPACT>
-__device__ __forceinline__ void cz_coefs(const Coupling<T>& k, uint32_t f, const T* sal,
-                                         const T* sah, T* al, T* ah) {
-#pragma unroll
-  for (int a = 0; a < DIM; ++a) {
-    if constexpr (COMPACT) {
-      al[a] = ((f >> (NB_DN + a)) & 1u) ? k.coef : (T)0;
-      ah[a] = ((f >> a) & 1u) ? k.coef : (T)0;
-    } else {
-      al[a] = sal[a];
-      ah[a] = sah[a];
-    }
-  }
-}
-
-// smooth(l, c) over the level (mgpcg.py:104-109)
-template <typename T, int DIM, bool COMPACT>
-__device__ void cz_half_t(const Geo& g, const LevelPtrs<T>& P, const Coupling<T>& k, int c) {
-  const int n = g.size;
-  constexpr int NS = cz_slots<COMPACT>();
-  for (int b = 0; b < n; b += NS * COARSE_THREADS) {
-    CzOps<T, DIM, COMPACT> v[NS];
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const int t = b + s * COARSE_THREADS + (int)threadIdx.x;
-      v[s].gt = MG_SOLID;
-      if (t < n) cz_gather<T, DIM, COMPACT>(g, P, c, t, false, v[s]);
-    }
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const int t = b + s * COARSE_THREADS + (int)threadIdx.x;
-      if (v[s].gt != MG_FLUID) continue;
-      T al[DIM], ah[DIM];
-      cz_coefs<T, DIM, COMPACT>(k, v[s].f, v[s].al, v[s].ah, al, ah);
-      T sm = nsum_vals<T, DIM>(al, ah, v[s].zl, v[s].zh);
-      T num = v[s].rv - sm;
-      P.z[c][t] = num / v[s].ad;
-    }
-  }
-  __syncthreads();
-}
-template <typename T, int DIM>
-__device__ void cz_half(const Geo& g, const LevelPtrs<T>& P, const Coupling<T>& k, int c) {
-  if (k.uniform) cz_half_t<T, DIM, true>(g, P, k, c);
-  else cz_half_t<T, DIM, false>(g, P, k, c);
-}
-
-// z.fill(0); smooth(l, 0): z0 = r0 / Adiag0 on FLUID, 0 elsewhere, and z1 = 0
-// (the smooth(l, 1) that follows rewrites every colour-1 FLUID value)
 template <typename T>
-__device__ void cz_first(const Geo& g, const LevelPtrs<T>& P) {
-  const int n = g.size;
-  for (int b = 0; b < n; b += CZ_SLOTS * COARSE_THREADS) {
-    int gt[CZ_SLOTS];
-    T rv[CZ_SLOTS], ad[CZ_SLOTS];
-#pragma unroll
-    for (int s = 0; s < CZ_SLOTS; ++s) {
-      const int t = b + s * COARSE_THREADS + (int)threadIdx.x;
-      gt[s] = MG_SOLID;
-      if (t < n) {
-        gt[s] = P.gt[0][t];
-        rv[s] = P.r[0][t];
-        ad[s] = P.Adiag[0][t];
-      }
-    }
-#pragma unroll
-    for (int s = 0; s < CZ_SLOTS; ++s) {
-      const int t = b + s * COARSE_THREADS + (int)threadIdx.x;
-      if (t >= n) continue;
-      P.z[0][t] = gt[s] == MG_FLUID ? rv[s] / ad[s] : (T)0;
-      P.z[1][t] = (T)0;
-    }
-  }
-  __syncthreads();
-}
-
-template <typename T>
-__device__ void cz_zero(const Geo& g, const LevelPtrs<T>& P) {
-  for (int t = threadIdx.x; t < g.size; t += COARSE_THREADS) zero_slot<T>(P, t);
-  __syncthreads();
-}
-
-// restrict(l) (mgpcg.py:111-118) into the coarser level's r: the residual of
-// every fine cell (0 off FLUID) into `res` (two colour arrays of the fine
-// level's size), then every interior coarse cell sums its eight children in
-// lexicographic order (adding a 0 leaves the sum unchanged, as skipping a
-// non-FLUID child does: the sum starts at +0 and never becomes -0)
-template <typename T, int DIM, bool COMPACT>
-__device__ void cz_residuals(const Geo& gf, const LevelPtrs<T>& F, const Coupling<T>& k,
-                             T* const* res) {
-  const int n = gf.size;
+__device__ __forceinline__ CzLevel<T> cz_level(unsigned char* b, int n) {
+  const int vb = lds_align(n * (int)sizeof(T)), wb = lds_align(2 * n);
+  CzLevel<T> v;
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
-    constexpr int NS = cz_slots<COMPACT>();
-    for (int b = 0; b < n; b += NS * COARSE_THREADS) {
-    CzOps<T, DIM, COMPACT> v[NS];
-#pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        const int t = b + s * COARSE_THREADS + (int)threadIdx.x;
-        v[s].gt = MG_SOLID;
-        if (t < n) cz_gather<T, DIM, COMPACT>(gf, F, c, t, true, v[s]);
-      }
-#pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        const int t = b + s * COARSE_THREADS + (int)threadIdx.x;
-        if (t >= n) continue;
-        T rr = (T)0;
-        if (v[s].gt == MG_FLUID) {
-          T al[DIM], ah[DIM];
-          cz_coefs<T, DIM, COMPACT>(k, v[s].f, v[s].al, v[s].ah, al, ah);
-          T Az = v[s].ad * v[s].own;
-          T ns = nsum_vals<T, DIM>(al, ah, v[s].zl, v[s].zh);
-          Az = Az + ns;
-          rr = v[s].rv - Az;
-        }
-        res[c][t] = rr;
-      }
-    }
+    v.z[c] = (T*)(b + c * vb);
+    v.res[c] = (T*)(b + (2 + c) * vb);
+    v.r[c] = (T*)(b + (4 + c) * vb);
+    v.list[c] = (uint16_t*)(b + 6 * vb + c * wb);
   }
-  __syncthreads();
+  return v;
 }
 
+// One owned slot: its place (slot | parity q << 16) and its operator row.
 template <typename T, int DIM>
-__device__ void cz_restrict(const Geo& gf, const LevelPtrs<T>& F, const Coupling<T>& k,
-                            const Geo& gc, T* rc0, T* rc1, T* const* res) {
-  if (k.uniform) cz_residuals<T, DIM, true>(gf, F, k, res);
-  else cz_residuals<T, DIM, false>(gf, F, k, res);
-  const int nc = gc.size;
-  for (int tc = threadIdx.x; tc < nc; tc += COARSE_THREADS) {
-#pragma unroll
-    for (int cc = 0; cc < 2; ++cc) {
-      const Slot s = decode(gc, tc, cc);
-      if (!s.interior) continue;
-      T v[8];
-      int nch = 0;
-#pragma unroll
-      for (int o0 = 0; o0 < (DIM == 3 ? 2 : 1); ++o0)
-#pragma unroll
-        for (int o1 = 0; o1 < 2; ++o1)
-#pragma unroll
-          for (int o2 = 0; o2 < 2; ++o2) {
-            const int i = (DIM == 3) ? 2 * s.i + o0 : 0;
-            const int j = 2 * s.j + o1, kk = 2 * s.k + o2;
-            v[nch++] = res[colour_of(i, j, kk)][slot_of(gf, i, j, kk)];
-          }
-      T sum = (T)0;
-#pragma unroll
-      for (int o = 0; o < (DIM == 3 ? 8 : 4); ++o) sum = sum + v[o];
-      (cc ? rc1 : rc0)[tc] = sum;
-    }
-  }
-  __syncthreads();
-}
+struct CzRow {
+  int p;
+  bool on;
+  T r, ad, y, al[DIM], ah[DIM];  // y = 1 / ad, or 0 where cz_div takes the plain division
+  __device__ __forceinline__ int t() const { return p & 0xffff; }
+};
 
-// coarse_pre / coarse_bottom / coarse_post on the LDS image
+// num / ad, correctly rounded, from y = 1 / ad correctly rounded: two
+// residual corrections of num * y, each exact to a rounding (Markstein,
+// "Computation of elementary functions on the IBM RISC System/6000 processor",
+// 1990).  5 instructions in place of the general division's 12; outside the
+// exponents where no step can underflow or overflow, the division itself.
 template <typename T, int DIM>
-__device__ void cz_pre(const Geo& g, const LevelPtrs<T>& P, int nu) {
-  if (nu <= 0) {
-    cz_zero<T>(g, P);
-    return;
-  }
-  const Coupling<T> k = coupling(P);
-  cz_first<T>(g, P);
-  cz_half<T, DIM>(g, P, k, 1);
-  for (int i = 1; i < nu; ++i) {
-    cz_half<T, DIM>(g, P, k, 0);
-    cz_half<T, DIM>(g, P, k, 1);
-  }
+__device__ __forceinline__ T cz_div(T num, const CzRow<T, DIM>& w) {
+  T q = num * w.y;
+  q = fmaf(fmaf(-w.ad, q, num), w.y, q);
+  q = fmaf(fmaf(-w.ad, q, num), w.y, q);
+  const uint32_t e = (__float_as_uint(num) >> 23) & 255u;
+  if (e - 47u >= 160u || w.y == (T)0) q = num / w.ad;  // |num| outside [2^-80, 2^80)
+  return q;
 }
-
-template <typename T, int DIM>
-__device__ void cz_bottom(const Geo& g, const LevelPtrs<T>& P, int bottom) {
-  const int half = bottom / 2;
-  if (half <= 0) {
-    cz_zero<T>(g, P);
-    return;
-  }
-  const Coupling<T> k = coupling(P);
-  cz_first<T>(g, P);
-  cz_half<T, DIM>(g, P, k, 1);
-  for (int i = 1; i < half; ++i) {
-    cz_half<T, DIM>(g, P, k, 0);
-    cz_half<T, DIM>(g, P, k, 1);
-  }
-  for (int i = 0; i < half; ++i) {
-    cz_half<T, DIM>(g, P, k, 1);
-    cz_half<T, DIM>(g, P, k, 0);
-  }
-}
-
-// prolongate(l) (mgpcg.py:120-123) on colour 0: the smooth(l, 1) that follows
-// reads these values, each z0 + z_coarse[parent] formed as the reference
-// forms it, and rewrites every colour-1 FLUID value without reading it.
-// (Colour-1 cells that are not FLUID keep z unprolongated, as do those of
-// the global-memory form: no FLUID result reads them -- their couplings are
-// 0 and the children of a cell that is not FLUID are not FLUID.)
 template <typename T>
-__device__ void cz_prolong0(const Geo& g, const Geo& gc, const LevelPtrs<T>& P, const T* zc0,
-                            const T* zc1) {
-  const int n = g.size;
-  for (int b = 0; b < n; b += CZ_SLOTS * COARSE_THREADS) {
-    T zv[CZ_SLOTS], pv[CZ_SLOTS];
-    bool in[CZ_SLOTS];
+__device__ __forceinline__ T cz_reciprocal(T ad) {
+  const uint32_t e = (__float_as_uint(ad) >> 23) & 255u;
+  return e - 87u < 80u ? (T)1 / ad : (T)0;  // |ad| in [2^-40, 2^40)
+}
+
+// the lane's rows of colour c of a level (not r)
+template <typename T, int DIM, int NS>
+__device__ __forceinline__ void cz_rows(const Geo& g, const LevelPtrs<T>& P, const Coupling<T>& k,
+                                        const uint16_t* list, int n, int c,
+                                        CzRow<T, DIM>* w) {
+  // a slot whose neighbours lie inside the arrays, for lanes without a row
+  const int safe = (DIM == 3 ? g.sx : 0) + g.W + 1;
+  uint32_t f[NS];
 #pragma unroll
-    for (int s = 0; s < CZ_SLOTS; ++s) {
-      const int t = b + s * COARSE_THREADS + (int)threadIdx.x;
-      in[s] = false;
-      if (t >= n) continue;
-      const Slot sl = decode(g, t, 0);
-      if (!sl.interior) continue;
-      in[s] = true;
-      const int pi = sl.i >> 1, pj = sl.j >> 1, pk = sl.k >> 1;
-      const int ps = slot_of(gc, pi, pj, pk);
-      pv[s] = colour_of(pi, pj, pk) ? zc1[ps] : zc0[ps];
-      zv[s] = P.z[0][t];
-    }
+  for (int s = 0; s < NS; ++s) {
+    const int i = s * COARSE_THREADS + (int)threadIdx.x;
+    w[s].on = i < n;
+    const int t = w[s].on ? (int)list[i] : safe;
+    const int q = row_q(g, t, c);
+    w[s].p = t | (q << 16);
+    w[s].ad = ldgi(P.Adiag[c], t);
+    if (k.uniform) {
+      f[s] = ldgi(P.nb[c], t);
+    } else {
+      const Nbr<DIM> nb = neighbours_clamped<DIM>(g, t, q);
 #pragma unroll
-    for (int s = 0; s < CZ_SLOTS; ++s) {
-      const int t = b + s * COARSE_THREADS + (int)threadIdx.x;
-      if (in[s]) P.z[0][t] = zv[s] + pv[s];
+      for (int a = 0; a < DIM; ++a) {
+        w[s].al[a] = ldgi(P.Ax[a][c ^ 1], nb.lo[a]);
+        w[s].ah[a] = ldgi(P.Ax[a][c], t);
+      }
     }
+  }
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    if (k.uniform) {
+#pragma unroll
+      for (int a = 0; a < DIM; ++a) {
+        w[s].al[a] = ((f[s] >> (NB_DN + a)) & 1u) ? k.coef : (T)0;
+        w[s].ah[a] = ((f[s] >> a) & 1u) ? k.coef : (T)0;
+      }
+    }
+    w[s].ad = w[s].on ? w[s].ad : (T)1;
+    w[s].y = cz_reciprocal(w[s].ad);
+  }
+}
+
+// NS: the lane's rows.  With several, their neighbours' addresses would take
+// more registers than there are: they are formed at each use.
+template <typename T, int DIM, int NS>
+__device__ __forceinline__ void cz_gather(const Geo& g, const T* zo, const CzRow<T, DIM>& w, T* zl,
+                                          T* zh) {
+  int p = w.p;
+  if constexpr (NS > 1) MG_HERE(p);
+  const Nbr<DIM> n = neighbours<DIM>(g, p & 0xffff, p >> 16);
+#pragma unroll
+  for (int a = 0; a < DIM; ++a) {
+    zl[a] = zo[n.lo[a]];
+    zh[a] = zo[n.hi[a]];
+  }
+}
+
+// smooth(l, c) (mgpcg.py:104-109); FIRST: from z = 0, without reading it
+template <typename T, int DIM, int NS, bool FIRST = false>
+__device__ __forceinline__ void cz_half(const Geo& g, const CzLevel<T>& v, const CzRow<T, DIM>* w,
+                                        int n, int c) {
+  T zl[NS][DIM], zh[NS][DIM];
+  if constexpr (!FIRST) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+      if (s * COARSE_THREADS < n) cz_gather<T, DIM, NS>(g, v.z[c ^ 1], w[s], zl[s], zh[s]);
+  }
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    if (s * COARSE_THREADS >= n) break;
+    T num = w[s].r;
+    if constexpr (!FIRST) {
+      const T sm = nsum_vals<T, DIM>(w[s].al, w[s].ah, zl[s], zh[s]);
+      num = w[s].r - sm;
+    }
+    if (w[s].on) v.z[c][w[s].t()] = cz_div<T, DIM>(num, w[s]);
   }
   __syncthreads();
 }
 
+// the residuals r - A z of both colours (restrict, mgpcg.py:111-118)
+template <typename T, int DIM, int NS>
+__device__ __forceinline__ void cz_residuals(const Geo& g, const CzLevel<T>& v,
+                                             const CzRow<T, DIM> (*w)[NS], const int* n) {
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      if (s * COARSE_THREADS >= n[c]) break;
+      const CzRow<T, DIM>& x = w[c][s];
+      T zl[DIM], zh[DIM];
+      cz_gather<T, DIM, NS>(g, v.z[c ^ 1], x, zl, zh);
+      T Az = x.ad * v.z[c][x.t()];
+      const T ns = nsum_vals<T, DIM>(x.al, x.ah, zl, zh);
+      Az = Az + ns;
+      if (x.on) v.res[c][x.t()] = x.r - Az;
+    }
+  __syncthreads();
+}
+
+// a coarse row's right-hand side: its children's residuals in lexicographic
+// order (a child that is not FLUID has 0, which leaves the sum unchanged)
 template <typename T, int DIM>
-__device__ void cz_post(const Geo& g, const Geo& gc, const LevelPtrs<T>& P, T* const* zc,
-                        int nu) {
-  if (nu <= 0) {
-    coarse_post<T, DIM>(g, gc, P, zc, nu);
-    return;
+__device__ __forceinline__ void cz_sum(const Geo& gf, const CzLevel<T>& F, const Geo& g, int c,
+                                       CzRow<T, DIM>& w) {
+  const Slot s = decode(g, w.t(), c);
+  const bool in = w.on;
+  T sum = (T)0;
+#pragma unroll
+  for (int o0 = 0; o0 < (DIM == 3 ? 2 : 1); ++o0)
+#pragma unroll
+    for (int o1 = 0; o1 < 2; ++o1)
+#pragma unroll
+      for (int o2 = 0; o2 < 2; ++o2) {
+        const int i = (DIM == 3) ? 2 * s.i + o0 : 0;
+        const int j = 2 * s.j + o1, k = 2 * s.k + o2;
+        sum = sum + F.res[colour_of(i, j, k)][in ? slot_of(gf, i, j, k) : 0];
+      }
+  w.r = sum;
+}
+
+// smoothing before the restriction (mgpcg.py:126-131); z holds 0
+template <typename T, int DIM, int NS>
+__device__ __forceinline__ void cz_pre(const Geo& g, const CzLevel<T>& v,
+                                       const CzRow<T, DIM> (*w)[NS], const int* n, int steps) {
+  for (int i = 0; i < steps; ++i) {
+    if (i == 0) cz_half<T, DIM, NS, true>(g, v, w[0], n[0], 0);
+    else cz_half<T, DIM, NS>(g, v, w[0], n[0], 0);
+    cz_half<T, DIM, NS>(g, v, w[1], n[1], 1);
   }
-  const Coupling<T> k = coupling(P);
-  cz_prolong0<T>(g, gc, P, zc[0], zc[1]);
-  cz_half<T, DIM>(g, P, k, 1);
-  cz_half<T, DIM>(g, P, k, 0);
-  for (int i = 1; i < nu; ++i) {
-    cz_half<T, DIM>(g, P, k, 1);
-    cz_half<T, DIM>(g, P, k, 0);
+}
+template <typename T, int DIM, int NS>
+__device__ __forceinline__ void cz_back(const Geo& g, const CzLevel<T>& v,
+                                        const CzRow<T, DIM> (*w)[NS], const int* n, int steps) {
+  for (int i = 0; i < steps; ++i) {
+    cz_half<T, DIM, NS>(g, v, w[1], n[1], 1);
+    cz_half<T, DIM, NS>(g, v, w[0], n[0], 0);
   }
 }
 
-// LDS image of one system's coarse levels: per level the z, r and Adiag
-// colour arrays, the cell types, the coupling flags and the coupling range.
-// The stored couplings (Ax) of a level without uniform couplings stay in
-// global memory.
-constexpr int COARSE_LDS_BYTES = 160 * 1024;
-__host__ __device__ constexpr int lds_align(int b) { return (b + 15) & ~15; }
-__host__ __device__ constexpr int coarse_image_bytes(int size, int esz) {
-  return 6 * lds_align(size * esz) + 2 * lds_align(size) + 2 * lds_align(2 * size) +
-         lds_align((int)sizeof(LevelMeta));
+// prolongate(l) (mgpcg.py:120-123) and the smoothing after it (:143-147).  The
+// smooth(l, 1) that follows rewrites every colour-1 value, so with smoothing
+// only colour 0 is prolongated.
+template <typename T, int DIM, int NS>
+__device__ __forceinline__ void cz_post(const Geo& g, const CzLevel<T>& v,
+                                        const CzRow<T, DIM> (*w)[NS], const int* n, const Geo& gc,
+                                        const CzLevel<T>& C, int nu) {
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    if (c == 1 && nu > 0) break;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      if (s * COARSE_THREADS >= n[c]) break;
+      if (!w[c][s].on) continue;
+      const int t = w[c][s].t();
+      const Slot sl = decode(g, t, c);
+      const int pi = sl.i >> 1, pj = sl.j >> 1, pk = sl.k >> 1;
+      const T zc = C.z[colour_of(pi, pj, pk)][slot_of(gc, pi, pj, pk)];
+      v.z[c][t] = v.z[c][t] + zc;
+    }
+  }
+  __syncthreads();
+  cz_back<T, DIM, NS>(g, v, w, n, nu);
 }
-// the restriction's fine residuals (two colour arrays of the largest level
-// that restricts), after the levels' images
-__host__ __device__ constexpr int coarse_scratch_bytes(int size, int esz) {
-  return 2 * lds_align(size * esz);
+
+// Levels d0 .. d0 + nlev - 1 of one system on the LDS image `img`; cnt: LDS,
+// two counters per level.
+template <typename T, int DIM>
+__device__ void cz_vcycle(const LevelDesc<T>* descs, int d0, int nlev, int nu, int bottom,
+                          unsigned char* img, unsigned* cnt) {
+  constexpr int NS = cz_slots<DIM>();
+  // list every level's FLUID slots, and zero its z and residuals
+  if ((int)threadIdx.x < 2 * nlev) cnt[threadIdx.x] = 0;
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  int off = 0;
+  for (int k = 0; k < nlev; ++k) {
+    const LevelDesc<T>& D = descs[d0 + k];
+    const int n = D.g.size;
+    const CzLevel<T> v = cz_level<T>(img + off, n);
+    off += coarse_image_bytes(n, (int)sizeof(T));
+    constexpr int NB = 2 * CZ_MAX_SLOTS / COARSE_THREADS;
+    int gt[NB];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {  // every cell type before the first ballot
+      const int t = (u >> 1) * COARSE_THREADS + (int)threadIdx.x;
+      gt[u] = t < n ? (int)ldgi(D.P.gt[u & 1], t) : MG_SOLID;
+    }
+    struct alignas(16) Zero4 { T v[16 / sizeof(T)]; };
+    Zero4* z4 = (Zero4*)v.z[0];  // z[0], z[1], res[0], res[1] are contiguous
+    const int n4 = 4 * lds_align(n * (int)sizeof(T)) / 16;
+    for (int i = threadIdx.x; i < n4; i += COARSE_THREADS) z4[i] = Zero4{};
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      if ((u >> 1) * COARSE_THREADS >= n) break;
+      const unsigned long long m = __ballot(gt[u] == MG_FLUID);
+      unsigned at = 0;
+      if (lane == 0 && m != 0) at = atomicAdd(cnt + 2 * k + (u & 1), (unsigned)__builtin_popcountll(m));
+      at = (unsigned)MG_READLANE((int)at, 0);
+      if (gt[u] == MG_FLUID)
+        v.list[u & 1][at + __builtin_popcountll(m & ((1ull << lane) - 1ull))] =
+            (uint16_t)((u >> 1) * COARSE_THREADS + (int)threadIdx.x);
+    }
+  }
+  __syncthreads();
+  auto count = [&](int k, int* n) {
+    n[0] = MG_UNIFORM((int)cnt[2 * k]);
+    n[1] = MG_UNIFORM((int)cnt[2 * k + 1]);
+  };
+  auto offset = [&](int k) {
+    int o = 0;
+    for (int j = 0; j < k; ++j) o += coarse_image_bytes(descs[d0 + j].g.size, (int)sizeof(T));
+    return o;
+  };
+  // the first two levels' rows stay in registers; the levels below (and only
+  // they) load theirs at each visit
+  const Geo gA = descs[d0].g;
+  const LevelPtrs<T> PA = descs[d0].P;
+  const CzLevel<T> vA = cz_level<T>(img, gA.size);
+  int nA[2];
+  count(0, nA);
+  CzRow<T, DIM> A[2][NS];
+  {
+    const Coupling<T> kc = coupling_g(PA);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      cz_rows<T, DIM, NS>(gA, PA, kc, vA.list[c], nA[c], c, A[c]);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) A[c][s].r = ldgi(PA.r[c], A[c][s].t());
+    }
+  }
+  if (nlev == 1) {
+    cz_pre<T, DIM, NS>(gA, vA, A, nA, bottom / 2);
+    cz_back<T, DIM, NS>(gA, vA, A, nA, bottom / 2);
+  } else {
+    const Geo gB = descs[d0 + 1].g;
+    const CzLevel<T> vB = cz_level<T>(img + offset(1), gB.size);
+    int nB[2];
+    count(1, nB);
+    CzRow<T, DIM> B[2][1];
+    {
+      const LevelPtrs<T> PB = descs[d0 + 1].P;
+      const Coupling<T> kc = coupling_g(PB);
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        cz_rows<T, DIM, 1>(gB, PB, kc, vB.list[c], nB[c], c, B[c]);
+    }
+    cz_pre<T, DIM, NS>(gA, vA, A, nA, nu);
+    cz_residuals<T, DIM, NS>(gA, vA, A, nA);
+    cz_sum<T, DIM>(gA, vA, gB, 0, B[0][0]);
+    cz_sum<T, DIM>(gA, vA, gB, 1, B[1][0]);
+    if (nlev == 2) {
+      cz_pre<T, DIM, 1>(gB, vB, B, nB, bottom / 2);
+      cz_back<T, DIM, 1>(gB, vB, B, nB, bottom / 2);
+    } else {
+      cz_pre<T, DIM, 1>(gB, vB, B, nB, nu);
+      cz_residuals<T, DIM, 1>(gB, vB, B, nB);
+      for (int k = 2; k < 2 * nlev - 3; ++k) {  // down to the bottom, up to level 2
+        const bool down = k < nlev;
+        const int l = down ? k : 2 * nlev - 2 - k;
+        const LevelDesc<T>& D = descs[d0 + l];
+        const Geo g = D.g;
+        const CzLevel<T> v = cz_level<T>(img + offset(l), g.size);
+        int n[2];
+        count(l, n);
+        CzRow<T, DIM> X[2][1];
+        const Coupling<T> kc = coupling_g(D.P);
+        if (down) {
+          const Geo gf = descs[d0 + l - 1].g;
+          const CzLevel<T> F = cz_level<T>(img + offset(l - 1), gf.size);
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            cz_rows<T, DIM, 1>(g, D.P, kc, v.list[c], n[c], c, X[c]);
+            cz_sum<T, DIM>(gf, F, g, c, X[c][0]);
+            if (X[c][0].on) v.r[c][X[c][0].t()] = X[c][0].r;
+          }
+          if (l == nlev - 1) {
+            cz_pre<T, DIM, 1>(g, v, X, n, bottom / 2);
+            cz_back<T, DIM, 1>(g, v, X, n, bottom / 2);
+          } else {
+            cz_pre<T, DIM, 1>(g, v, X, n, nu);
+            cz_residuals<T, DIM, 1>(g, v, X, n);
+          }
+        } else {
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            cz_rows<T, DIM, 1>(g, D.P, kc, v.list[c], n[c], c, X[c]);
+            X[c][0].r = v.r[c][X[c][0].t()];
+          }
+          const CzLevel<T> C = cz_level<T>(img + offset(l + 1), D.gc.size);
+          cz_post<T, DIM, 1>(g, v, X, n, D.gc, C, nu);
+        }
+      }
+      const Geo g2 = descs[d0 + 2].g;
+      cz_post<T, DIM, 1>(gB, vB, B, nB, g2, cz_level<T>(img + offset(2), g2.size), nu);
+    }
+    cz_post<T, DIM, NS>(gA, vA, A, nA, gB, vB, nu);
+  }
+  // the finer level's prolongation reads the first coarse level's z
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+      if (A[c][s].on) stgi(PA.z[c], A[c][s].t(), vA.z[c][A[c][s].t()]);
 }
 
 // One workgroup per item: item.desc = the system's LevelDesc of its first
 // coarse level, item.block0 = number of levels from there to the bottom
-// (a system's LevelDescs are contiguous).  With USE_LDS every per-slot array
-// the V-cycle reads is copied into LDS once (the host checks that the
-// levels' coarse_image_bytes and the restriction's coarse_scratch_bytes fit
-// COARSE_LDS_BYTES), the V-cycle runs on the copy in the multi-slot phases
-// above, and z of every level and the restricted r of the levels below the
-// first are copied back at the end.  Without, the slot functions of the
-// global-memory form run on the levels in place.
+// (a system's LevelDescs are contiguous).  With USE_LDS the levels run on LDS
+// (cz_vcycle; the host checks that the levels' coarse_image_bytes fit
+// COARSE_LDS_BYTES and the first level CZ_MAX_SLOTS).  Without, the slot
+// functions of the global-memory form run on the levels in place.
 template <typename T, int DIM, bool USE_LDS>
 __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(const LevelDesc<T>* __restrict__ descs,
                                                            const Item* __restrict__ items,
-                                                           int nitems, int nu, int bottom) {
+                                                           int nitems, Item one, int nu,
+                                                           int bottom) {
   if ((int)blockIdx.x >= nitems) return;
-  const int d0 = items[blockIdx.x].desc;
-  const int nlev = items[blockIdx.x].block0;
+  if (nitems > 1) one = items[blockIdx.x];
+  const int d0 = MG_UNIFORM(one.desc);
+  const int nlev = MG_UNIFORM(one.block0);
   if (descs[d0].st->done) return;
-  __shared__ alignas(16) unsigned char img[USE_LDS ? COARSE_LDS_BYTES : 16];
-  // the operator and vectors of coarse level k as the V-cycle sees them
-  auto lv = [&](int k) -> LevelPtrs<T> {
-    LevelPtrs<T> P = descs[d0 + k].P;
-    if constexpr (USE_LDS) {
-      int off = 0;
-      for (int j = 0; j < k; ++j) off += coarse_image_bytes(descs[d0 + j].g.size, (int)sizeof(T));
-      const int n = descs[d0 + k].g.size;
-      const int vb = lds_align(n * (int)sizeof(T)), bb = lds_align(n), wb = lds_align(2 * n);
-      unsigned char* b = img + off;
-      P.z[0] = (T*)(b + 0 * vb);
-      P.z[1] = (T*)(b + 1 * vb);
-      P.r[0] = (T*)(b + 2 * vb);
-      P.r[1] = (T*)(b + 3 * vb);
-      P.Adiag[0] = (const T*)(b + 4 * vb);
-      P.Adiag[1] = (const T*)(b + 5 * vb);
-      P.gt[0] = (const int8_t*)(b + 6 * vb);
-      P.gt[1] = (const int8_t*)(b + 6 * vb + bb);
-      P.nb[0] = (const uint16_t*)(b + 6 * vb + 2 * bb);
-      P.nb[1] = (const uint16_t*)(b + 6 * vb + 2 * bb + wb);
-      if (P.meta != nullptr) P.meta = (const LevelMeta*)(b + 6 * vb + 2 * bb + 2 * wb);
-    }
-    return P;
-  };
   if constexpr (USE_LDS) {
-    for (int k = 0; k < nlev; ++k) {
-      const LevelPtrs<T> G = descs[d0 + k].P;
-      const LevelPtrs<T> P = lv(k);
-      const int n = descs[d0 + k].g.size;
-      const bool flags = G.meta != nullptr;
-      // all loads of a lane's slots in flight before the first LDS store
-      for (int b = 0; b < n; b += CZ_SLOTS * COARSE_THREADS) {
-        T rv[CZ_SLOTS][2], ad[CZ_SLOTS][2];
-        int8_t gt[CZ_SLOTS][2];
-        uint16_t f[CZ_SLOTS][2];
-#pragma unroll
-        for (int s = 0; s < CZ_SLOTS; ++s) {
-          const int t = b + s * COARSE_THREADS + (int)threadIdx.x;
-          if (t >= n) continue;
-#pragma unroll
-          for (int c = 0; c < 2; ++c) {
-            rv[s][c] = ldgi(G.r[c], t);
-            ad[s][c] = ldgi(G.Adiag[c], t);
-            gt[s][c] = ldgi(G.gt[c], t);
-            f[s][c] = flags ? ldgi(G.nb[c], t) : (uint16_t)0;
-          }
-        }
-#pragma unroll
-        for (int s = 0; s < CZ_SLOTS; ++s) {
-          const int t = b + s * COARSE_THREADS + (int)threadIdx.x;
-          if (t >= n) continue;
-#pragma unroll
-          for (int c = 0; c < 2; ++c) {
-            P.r[c][t] = rv[s][c];
-            const_cast<T*>(P.Adiag[c])[t] = ad[s][c];
-            const_cast<int8_t*>(P.gt[c])[t] = gt[s][c];
-            if (flags) const_cast<uint16_t*>(P.nb[c])[t] = f[s][c];
-          }
-        }
-      }
-      if (flags && threadIdx.x == 0) *const_cast<LevelMeta*>(P.meta) = *G.meta;
-    }
-    __syncthreads();
-  }
-  if constexpr (USE_LDS) {
-    int off = 0;
-    for (int j = 0; j < nlev; ++j) off += coarse_image_bytes(descs[d0 + j].g.size, (int)sizeof(T));
-    T* res[2];
-    res[0] = (T*)(img + off);
-    res[1] = (T*)(img + off + lds_align(descs[d0].g.size * (int)sizeof(T)));
-    // the geometry is read once per level into registers: a barrier orders
-    // memory, so fields read through the descriptor would be fetched again
-    // after every phase
-    for (int k = 0; k < nlev - 1; ++k) {
-      const Geo g = descs[d0 + k].g, gc = descs[d0 + k].gc;
-      const LevelPtrs<T> P = lv(k);
-      const LevelPtrs<T> C = lv(k + 1);
-      cz_pre<T, DIM>(g, P, nu);
-      cz_restrict<T, DIM>(g, P, coupling(P), gc, C.r[0], C.r[1], res);
-    }
-    {
-      const Geo gb = descs[d0 + nlev - 1].g;
-      cz_bottom<T, DIM>(gb, lv(nlev - 1), bottom);
-    }
-    for (int k = nlev - 2; k >= 0; --k) {
-      const Geo g = descs[d0 + k].g, gc = descs[d0 + k].gc;
-      const LevelPtrs<T> C = lv(k + 1);
-      cz_post<T, DIM>(g, gc, lv(k), C.z, nu);
-    }
+    __shared__ alignas(16) unsigned char img[COARSE_LDS_BYTES];
+    __shared__ unsigned cnt[2 * CZ_MAX_LEVELS];
+    cz_vcycle<T, DIM>(descs, d0, nlev, nu, bottom, img, cnt);
   } else {
     for (int k = 0; k < nlev - 1; ++k) {
       const LevelDesc<T>& D = descs[d0 + k];
-      const LevelPtrs<T> P = lv(k);
-      const LevelPtrs<T> C = lv(k + 1);
+      const LevelPtrs<T>& P = D.P;
+      const LevelPtrs<T>& C = descs[d0 + k + 1].P;
       coarse_pre<T, DIM>(D.g, P, nu);
       for (int tc = threadIdx.x; tc < D.gc.size; tc += COARSE_THREADS) {
         restrict_slot<T, DIM>(D.g, P, P.z, D.gc, C.r[0], C.r[1], 0, tc);
@@ -2334,27 +2324,10 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(const LevelDesc<T>* _
       }
       __syncthreads();
     }
-    coarse_bottom<T, DIM>(descs[d0 + nlev - 1].g, lv(nlev - 1), bottom);
+    coarse_bottom<T, DIM>(descs[d0 + nlev - 1].g, descs[d0 + nlev - 1].P, bottom);
     for (int k = nlev - 2; k >= 0; --k) {
       const LevelDesc<T>& D = descs[d0 + k];
-      const LevelPtrs<T> C = lv(k + 1);
-      coarse_post<T, DIM>(D.g, D.gc, lv(k), C.z, nu);
-    }
-  }
-  if constexpr (USE_LDS) {
-    // the finer level's prolongation reads the first coarse level's z; the
-    // other levels get z and r too, as the global-memory form leaves them
-    for (int k = 0; k < nlev; ++k) {
-      const LevelPtrs<T>& G = descs[d0 + k].P;
-      const LevelPtrs<T> P = lv(k);
-      const int n = descs[d0 + k].g.size;
-      for (int t = threadIdx.x; t < n; t += COARSE_THREADS) {
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          stgi(G.z[c], t, P.z[c][t]);
-          if (k > 0) stgi(G.r[c], t, P.r[c][t]);
-        }
-      }
+      coarse_post<T, DIM>(D.g, D.gc, D.P, descs[d0 + k + 1].P.z, nu);
     }
   }
 }

@@ -683,12 +683,17 @@ int engine_build_items(Engine* e) {
     x.desc = m * L + M.s->coarse_from;
     x.block0 = L - M.s->coarse_from;
     it.push_back(x);
-    long bytes = coarse_scratch_bytes(M.s->geo[M.s->coarse_from].size, (int)M.s->esz);
+    if (M.s->geo[M.s->coarse_from].size > CZ_MAX_SLOTS) {
+      e->coarse_lds = false;
+      continue;
+    }
+    long bytes = 0;
     for (int l = M.s->coarse_from; l < L; ++l)
       bytes += coarse_image_bytes(M.s->geo[l].size, (int)M.s->esz);
     if (bytes > COARSE_LDS_BYTES) e->coarse_lds = false;
   }
   e->st_coarse.n = (int)it.size() - e->st_coarse.off;
+  e->st_coarse.one = e->st_coarse.n > 0 ? it[e->st_coarse.off] : Item{0, 0};
   e->st_coarse.nblocks = e->st_coarse.n;
   // z.r after the V-cycle: fused into level 0's last half-sweep when level 0
   // is smoothed by the batched kernels, a plain dot otherwise
@@ -896,13 +901,13 @@ struct Sched {
         if (lds)
           hipLaunchKernelGGL((k_coarse<T, DIM, true>), dim3(e->st_coarse.n),
                              dim3(COARSE_THREADS), 0, e->stream, levels(e),
-                             (const Item*)(e->d_items + e->st_coarse.off), e->st_coarse.n, nu,
-                             e->bottom);
+                             (const Item*)(e->d_items + e->st_coarse.off), e->st_coarse.n,
+                             e->st_coarse.one, nu, e->bottom);
       }
       if (!lds)
         hipLaunchKernelGGL((k_coarse<T, DIM, false>), dim3(e->st_coarse.n), dim3(COARSE_THREADS),
                            0, e->stream, levels(e), (const Item*)(e->d_items + e->st_coarse.off),
-                           e->st_coarse.n, nu, e->bottom);
+                           e->st_coarse.n, e->st_coarse.one, nu, e->bottom);
     }
     for (int l = L - 2; l >= 0; --l) {
       if (tiled(e, l)) {

@@ -30,7 +30,6 @@
 #define HIP_SYMBOL(x) ((const void*)&(x))
 #define MG_GLOBAL
 #define MG_READLANE(v, l) (::hipemu::readlane_i((v), (l)))
-#define MG_UNIFORM(v) (v)
 #define MG_KEEP(x) ((void)(x))
 #define MG_KEEP4(a, b, c, d) ((void)(a), (void)(b), (void)(c), (void)(d))
 #define MG_KEEP6(a, b, c, d, e, f) ((void)(a), (void)(b), (void)(c), (void)(d), (void)(e), (void)(f))
