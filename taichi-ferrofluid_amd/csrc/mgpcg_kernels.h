@@ -147,6 +147,7 @@ struct LevelDesc {
   Geo g, gc;          // this level, next coarser level
   LevelPtrs<T> P, C;  // this level, next coarser level
   CGState* st;
+  DD* partials;            // the system's (SysDesc::partials)
   const LevelMeta* stats;  // the level's metadata, whatever P.meta says
 };
 
@@ -160,7 +161,7 @@ struct SysDesc {
   T* p[2][2];  // [iteration parity][colour]
   T* Ap[2];
   CGState* st;
-  DD* partials;  // one per 256-slot block of level 0 (a workgroup run's total in its first)
+  DD* partials;  // of dot products (RunSum): as many as level 0 has blocks
   int nparts;
   int coarse_from;  // first level handled by the single-workgroup coarse kernel
   int L;
@@ -498,9 +499,10 @@ __host__ __device__ constexpr int full_occupancy() {
 // Dot-product partials of one workgroup over a run of its virtual blocks in
 // one system: summed in registers and reduced over the workgroup once per run
 // (instead of once per virtual block) into the partial of the run's first
-// virtual block; the run's other virtual blocks get a zero partial, so every
-// partial of a system is written exactly once per launch.  run_mark and
-// run_flush are called by the whole workgroup (block-uniform control flow).
+// virtual block.  The finalize kernel reads those and no others: it derives
+// them from the launch's shape (run_first), at most one per workgroup where
+// level 0 has a block per 256 slots (66,000 at 256^3).  run_mark and run_flush
+// are called by the whole workgroup (block-uniform control flow).
 struct RunSum {
   DD acc = dd_zero();
   DD* dst = nullptr;  // receives the run's total
@@ -511,11 +513,11 @@ __device__ __forceinline__ void stg_dd(DD* p, DD v) {
 }
 __device__ __forceinline__ void run_mark(RunSum& r, DD* partials, int lb) {
   if (r.dst == nullptr) r.dst = partials + lb;
-  else if (threadIdx.x == 0) stg_dd(partials + lb, dd_zero());
 }
+template <int NT = BLOCK>
 __device__ __forceinline__ void run_flush(RunSum& r) {
   if (r.dst == nullptr) return;
-  const DD t = block_sum_dd<BLOCK>(r.acc);
+  const DD t = block_sum_dd<NT>(r.acc);
   if (threadIdx.x == 0) stg_dd(r.dst, t);
   r.acc = dd_zero();
   r.dst = nullptr;
@@ -1648,9 +1650,8 @@ __global__ void __launch_bounds__(TileShape<DIM>::NT) k_tile_pre(
   }
 }
 
-// prolongate(l) (mgpcg.py:120-123) and nu smoothing steps (:143-147).  L0:
-// without the last smooth(0, 0), which the kernel that also forms z.r does,
-// and with colour 1 only stored.
+// prolongate(l) (mgpcg.py:120-123) and nu smoothing steps (:143-147).  L0: with
+// reduce(z, r) (:171, :201), a partial per workgroup.
 template <typename T, int DIM, bool L0>
 __global__ void __launch_bounds__(TileShape<DIM>::NT) k_tile_post(
     const LevelDesc<T>* __restrict__ descs, Stage S, int nu) {
@@ -1659,10 +1660,12 @@ __global__ void __launch_bounds__(TileShape<DIM>::NT) k_tile_post(
   __shared__ T z[Ts::CELLS];
   __shared__ int any;
   ItemCache ic;
+  RunSum rs;
   int done = 1;
   Coupling<T> kc{false, (T)0};
   for (VBIter it = vb_begin(S.nblocks); it.vb < it.end; it.vb += it.step) {
     const bool fresh = item_at(S, it.vb, ic);
+    if (L0 && fresh) run_flush<Ts::NT>(rs);
     const LevelDesc<T>& D = descs[ic.desc];
     int oi, oj, ok;
     tile_origin<DIM>(D.g, it.vb - ic.block0, oi, oj, ok);
@@ -1698,6 +1701,7 @@ __global__ void __launch_bounds__(TileShape<DIM>::NT) k_tile_post(
       MG_KEEP(pv[s]);
     }
     if (done) continue;
+    if (L0) run_mark(rs, D.partials, it.vb - ic.block0);
     tile_couplings<T, DIM>(D.g, D.P, kc, f, v);
     __syncthreads();
     T own[2 * NS];
@@ -1715,7 +1719,7 @@ __global__ void __launch_bounds__(TileShape<DIM>::NT) k_tile_post(
     if (mine) any = 1;
     __syncthreads();
     if (any == 0) continue;
-    for (int h = 1; h <= 2 * nu - (L0 ? 1 : 0); ++h) {  // half-sweeps 1, 0, 1, ...
+    for (int h = 1; h <= 2 * nu; ++h) {  // half-sweeps 1, 0, 1, ...
       if (h & 1) {
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
@@ -1744,11 +1748,14 @@ __global__ void __launch_bounds__(TileShape<DIM>::NT) k_tile_post(
 #pragma unroll
     for (int s = 0; s < NS; ++s)
 #pragma unroll
-      for (int c = L0 ? 1 : 0; c < 2; ++c) {
+      for (int c = 0; c < 2; ++c) {
         const TileCell<T, DIM>& x = v[2 * s + c];
-        if (x.fluid && x.depth >= TILE_HALO) stgi(D.P.z[c], x.t, own[2 * s + c]);
+        if (!x.fluid || x.depth < TILE_HALO) continue;
+        stgi(D.P.z[c], x.t, own[2 * s + c]);
+        if (L0) rs.acc = dd_add(rs.acc, dd_prod(own[2 * s + c], x.r));
       }
   }
+  if (L0) run_flush<Ts::NT>(rs);
 }
 
 // restrict(l), child-parallel: 16 lanes per coarse slot -- 8 per coarse
@@ -2800,14 +2807,36 @@ __global__ void __launch_bounds__(BLOCK) k_dot_zr(const SysDesc<T, TX>* __restri
 // ---------------------------------------------------------------------------
 enum FinOp { FIN_INIT = 0, FIN_ALPHA = 1, FIN_RR = 2, FIN_TRUE = 3, FIN_BETA = 4 };
 
-// out (FIN_BETA only, may be NULL): the host's mapped readback slot; item i's
-// state after the step goes to out[i], done or not.
+// A launch of a kernel that left dot-product partials.
+struct Runs {
+  Stage S;
+  int grid;
+  bool levels;  // its items are level-0 LevelDescs, not systems
+};
+
+// Where workgroup w of a launch of G left its partial of the item that spans
+// virtual blocks [b0, e): its first block there, counted from b0; -1 if it has
+// none (vb_begin's ranges; per: blocks of a range).
+__device__ __forceinline__ int run_first(int w, int G, int per, int nblocks, int b0, int e) {
+  const int grp = G < 8 ? w : w & 7;
+  const int nx = G < 8 ? 1 : (G - grp + 7) >> 3;
+  const int end = min(nblocks, grp * per + per);
+  int first = grp * per + (G < 8 ? 0 : w >> 3);
+  if (first < b0) first += (b0 - first + nx - 1) / nx * nx;
+  return first < min(end, e) ? first - b0 : -1;
+}
+// R[0], and R[1] where its items are not all of them: the launches before.
+struct RunsPair {
+  Runs R[2];
+};
 template <typename T, typename TX, int OP>
 __global__ void __launch_bounds__(BLOCK) k_finalize(const SysDesc<T, TX>* __restrict__ sys,
                                                     const Item* __restrict__ items, int nitems,
-                                                    CGState* out) {
+                                                    Item one, RunsPair rp, CGState* out) {
   if ((int)blockIdx.x >= nitems) return;
-  const SysDesc<T, TX>& D = sys[items[blockIdx.x].desc];
+  if (nitems > 1) one = items[blockIdx.x];
+  const int m = MG_UNIFORM(one.desc);
+  const SysDesc<T, TX>& D = sys[m];
   CGState* st = D.st;
   if (st->done) {
     if (OP == FIN_BETA && out != nullptr && threadIdx.x == 0) {
@@ -2817,19 +2846,45 @@ __global__ void __launch_bounds__(BLOCK) k_finalize(const SysDesc<T, TX>* __rest
     return;
   }
   if (OP == FIN_TRUE && !st->pending_true) return;
-  // four independent accumulators: four partials per thread in flight
-  DD v0 = dd_zero(), v1 = dd_zero(), v2 = dd_zero(), v3 = dd_zero();
-  int i = threadIdx.x;
-  for (; i + 3 * BLOCK < D.nparts; i += 4 * BLOCK) {
-    const DD a = D.partials[i], b = D.partials[i + BLOCK];
-    const DD c = D.partials[i + 2 * BLOCK], d = D.partials[i + 3 * BLOCK];
-    v0 = dd_add(v0, a);
-    v1 = dd_add(v1, b);
-    v2 = dd_add(v2, c);
-    v3 = dd_add(v3, d);
+  // the system's virtual blocks in the launch that has it
+  __shared__ int span[3];
+  int which = rp.R[0].S.nitems > 0 ? 0 : 1, b0 = 0;
+  int e = rp.R[0].S.nblocks + rp.R[1].S.nblocks;
+  if (rp.R[0].S.nitems + rp.R[1].S.nitems > 1) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const Stage& S = rp.R[i].S;
+      const int want = rp.R[i].levels ? D.desc0 : m;
+      for (int k = threadIdx.x; k < S.nitems; k += BLOCK) {
+        const Item it = S.items[k];
+        if (it.desc != want) continue;
+        span[0] = i;
+        span[1] = it.block0;
+        span[2] = k + 1 < S.nitems ? S.items[k + 1].block0 : S.nblocks;
+      }
+    }
+    __syncthreads();
+    which = MG_UNIFORM(span[0]);
+    b0 = MG_UNIFORM(span[1]);
+    e = MG_UNIFORM(span[2]);
   }
-  for (; i < D.nparts; i += BLOCK) v0 = dd_add(v0, D.partials[i]);
-  const DD v = dd_add(dd_add(v0, v1), dd_add(v2, v3));
+  const int G = which ? rp.R[1].grid : rp.R[0].grid;
+  const int nblocks = which ? rp.R[1].S.nblocks : rp.R[0].S.nblocks;
+  const int per = (nblocks + min(G, 8) - 1) / min(G, 8);
+  // eight partials per thread in flight
+  DD v = dd_zero();
+  for (int w0 = threadIdx.x; w0 < G; w0 += 8 * BLOCK) {
+    DD p[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int w = w0 + u * BLOCK;
+      const int lb = w < G ? run_first(w, G, per, nblocks, b0, e) : -1;
+      p[u] = dd_zero();
+      if (lb >= 0) p[u] = DD{ldg(&D.partials[lb].hi), ldg(&D.partials[lb].lo)};
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v = dd_add(v, p[u]);
+  }
   const double tot = dd_value(block_sum_dd<BLOCK>(v));
   if (threadIdx.x != 0) return;
   if (OP == FIN_INIT) {

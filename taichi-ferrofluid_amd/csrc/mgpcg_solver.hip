@@ -159,6 +159,7 @@ LevelDesc<T> level_desc(const mgpcg_solver* s, int l) {
     d.C = d.P;
   }
   d.st = s->st;
+  d.partials = s->partials;
   d.stats = s->lv[l].meta;
   return d;
 }
@@ -764,6 +765,7 @@ inline Stage stage_of(const Engine* e, const Engine::StageRef& r) {
 }
 inline int grid_of(const Engine::StageRef& r) { return std::min(r.nblocks, g_max_grid); }
 
+
 // ---------------------------------------------------------------------------
 // iteration schedule, templated on hierarchy type T, x type TX and dimension
 // ---------------------------------------------------------------------------
@@ -815,12 +817,16 @@ struct Sched {
                          levels(e), stage_of(e, r));
     }
   }
-  // out: FIN_BETA's readback slot (see Engine::fused_gather)
+  // a, b: the stages of the launches that left the partials; out: FIN_BETA's
+  // readback slot (see Engine::fused_gather)
   template <int OP>
-  static void fin(Engine* e, const Engine::StageRef& r, CGState* out = nullptr) {
+  static void fin(Engine* e, const Engine::StageRef& r, const Engine::StageRef& a,
+                  bool levels = false, const Engine::StageRef& b = Engine::StageRef(),
+                  CGState* out = nullptr) {
     if (r.n == 0) return;
+    const RunsPair rp{{{stage_of(e, a), grid_of(a), levels}, {stage_of(e, b), grid_of(b), false}}};
     hipLaunchKernelGGL((k_finalize<T, TX, OP>), dim3(r.n), dim3(BLOCK), 0, e->stream, sys(e),
-                       (const Item*)(e->d_items + r.off), r.n, out);
+                       (const Item*)(e->d_items + r.off), r.n, r.one, rp, out);
   }
 
   // Whether level l runs as the two fused legs (an option that selects other
@@ -940,8 +946,9 @@ struct Sched {
         stage<ST_PROLONGATE>(e, S, l == 0);
       }
     }
-    // level 0's last half-sweep fused with reduce(z, r), or a plain dot
-    if (e->st_dot_fused.nblocks)
+    // level 0's last half-sweep fused with reduce(z, r) (its fused leg has
+    // both), or a plain dot
+    if (e->st_dot_fused.nblocks && !tiled(e, 0))
       hipLaunchKernelGGL((k_smooth0_dot<T, TX, DIM>), dim3(grid_of(e->st_dot_fused)),
                          dim3(BLOCK), 0, e->stream, sys(e), stage_of(e, e->st_dot_fused));
     if (e->st_dot_plain.nblocks)
@@ -958,7 +965,7 @@ struct Sched {
     if (e->st_init.nblocks) {
       hipLaunchKernelGGL((k_cg_init<T, TX>), dim3(grid_of(e->st_init)), dim3(BLOCK), 0,
                          e->stream, sys(e), stage_of(e, e->st_init));
-      fin<FIN_INIT>(e, e->fin_init);
+      fin<FIN_INIT>(e, e->fin_init, e->st_init);
       sync();
     }
     if (e->st_cg.nblocks) {
@@ -971,20 +978,22 @@ struct Sched {
         hipLaunchKernelGGL((k_cg_ap_only<T, TX, DIM>), dim3(grid_of(e->st_cg)), dim3(BLOCK), 0,
                            e->stream, sys(e), stage_of(e, e->st_cg));
       }
-      fin<FIN_ALPHA>(e, e->fin_cg);
+      fin<FIN_ALPHA>(e, e->fin_cg, e->st_cg);
       sync();
       hipLaunchKernelGGL((k_cg_xr<T, TX>), dim3(grid_of(e->st_cg)), dim3(BLOCK), 0, e->stream,
                          sys(e), stage_of(e, e->st_cg));
-      fin<FIN_RR>(e, e->fin_cg);
+      fin<FIN_RR>(e, e->fin_cg, e->st_cg);
       if (e->precision == MIXED) {
         hipLaunchKernelGGL((k_true_residual<T, TX, DIM>), dim3(grid_of(e->st_cg)), dim3(BLOCK),
                            0, e->stream, sys(e), stage_of(e, e->st_cg));
-        fin<FIN_TRUE>(e, e->fin_cg);
+        fin<FIN_TRUE>(e, e->fin_cg, e->st_cg);
       }
       sync();
     }
     vcycle(e, true);
-    fin<FIN_BETA>(e, e->fin_all, e->fused_gather);
+    const bool tiles = tiled(e, 0);
+    fin<FIN_BETA>(e, e->fin_all, tiles ? e->st_tile[0] : e->st_dot_fused, tiles, e->st_dot_plain,
+                  e->fused_gather);
     sync();
   }
 
@@ -1321,7 +1330,8 @@ void plan_pool(int dim, const int32_t* res, int n_levels, size_t esz, size_t xsz
   }
   P->ost = take(sizeof(CGState));
   P->nparts = nblk(g0.size);
-  P->opart = take(sizeof(DD) * P->nparts);
+  // a partial per block of level 0, of either kind
+  P->opart = take(sizeof(DD) * std::max(P->nparts, dim == 3 ? tile_count<3>(g0) : tile_count<2>(g0)));
   // the fused packing kernel's per-level table (same size for either precision)
   static_assert(sizeof(PackLevel<float>) == sizeof(PackLevel<double>), "");
   P->opack = take(sizeof(PackLevel<double>) * (size_t)n_levels);
