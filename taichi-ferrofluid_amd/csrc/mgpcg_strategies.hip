@@ -426,7 +426,10 @@ __global__ void k_add_c(long n, const int8_t* __restrict__ ct, float c, float* _
 
 // PotentialFunctionStrategy.build_b_kernel (potential_function.py:19-34).
 // in_domain(I) = all(I >= 0) and all(I + 1 <= res) on the fine res.
+template <int DIM>
 __global__ void k_potential_b(Shape s, Field chi, HField Hext, float* __restrict__ b) {
+  s.dim = DIM;
+  chi.s.dim = DIM;
   const long t = (long)blockIdx.x * SB + threadIdx.x;
   if (t >= s.cells()) return;
   int I[3];
@@ -458,8 +461,12 @@ __global__ void k_potential_b(Shape s, Field chi, HField Hext, float* __restrict
 
 // PotentialFunctionStrategy.build_A_kernel (potential_function.py:40-55) at
 // level l; `fine` is the fine shape used by in_domain at every level.
+template <int DIM>
 __global__ void k_potential_A(Shape s, Shape fine, int level, float dxl, Field chi,
                               float* __restrict__ Adiag, float* __restrict__ Ax) {
+  s.dim = DIM;
+  fine.dim = DIM;
+  chi.s.dim = DIM;
   const long t = (long)blockIdx.x * SB + threadIdx.x;
   if (t >= s.cells()) return;
   int I[3];
@@ -491,9 +498,13 @@ __global__ void k_potential_A(Shape s, Shape fine, int level, float dxl, Field c
 
 // SurfaceTensionStrategy.build_A_kernel (surface_tension.py:71-89) at level l;
 // the bounds I[k] +- 1 test the fine res at every level (surface_tension.py:82,86).
+template <int DIM>
 __global__ void k_surface_A(Shape s, Shape fine, int level, int d, Field phi, LS ls,
                             float inv_dt, float scale, float* __restrict__ Adiag,
                             float* __restrict__ Ax) {
+  s.dim = DIM;
+  fine.dim = DIM;
+  phi.s.dim = DIM;
   const long t = (long)blockIdx.x * SB + threadIdx.x;
   if (t >= s.cells()) return;
   int I[3];
@@ -523,7 +534,10 @@ __global__ void k_surface_A(Shape s, Shape fine, int level, int d, Field phi, LS
 }
 
 // SurfaceTension.calc_n (surface_tension.py:115-127): n as [cells, dim].
+template <int DIM>
 __global__ void k_calc_n(Shape s, int d, Field phi, float dx, float* __restrict__ n) {
+  s.dim = DIM;
+  phi.s.dim = DIM;
   const long t = (long)blockIdx.x * SB + threadIdx.x;
   if (t >= s.cells()) return;
   int I[3];
@@ -581,8 +595,10 @@ __device__ float sample_comp(const float* n, const Shape& s, int comp, const flo
   return a * (1.0f - q) + b * q;
 }
 
+template <int DIM>
 __global__ void k_calc_kappa(Shape s, const float* __restrict__ n, float dx,
                              float* __restrict__ kappa) {
+  s.dim = DIM;
   const long t = (long)blockIdx.x * SB + threadIdx.x;
   if (t >= s.cells()) return;
   int I[3];
@@ -601,9 +617,13 @@ __global__ void k_calc_kappa(Shape s, const float* __restrict__ n, float dx,
 }
 
 // SurfaceTensionStrategy.build_b_kernel (surface_tension.py:23-66).
+template <int DIM>
 __global__ void k_surface_b(Shape s, int d, Field u, Field phi, const float* __restrict__ kappa,
                             const float* __restrict__ n, LS ls, float dt, float dx, float dx2,
                             float sigma, float* __restrict__ b) {
+  s.dim = DIM;
+  u.s.dim = DIM;
+  phi.s.dim = DIM;
   const long t = (long)blockIdx.x * SB + threadIdx.x;
   if (t >= s.cells()) return;
   int I[3];
@@ -626,9 +646,12 @@ __global__ void k_surface_b(Shape s, int d, Field u, Field phi, const float* __r
   for (int a = 0; a < dim; ++a) nv[a] = n[t * dim + a];
   float Du = grad[0] * nv[0];
   for (int a = 1; a < dim; ++a) Du = Du + grad[a] * nv[a];
-  float D2[3][3];
+  float D2[3][3], own = 0.0f;
+  // sample(u, I + e1 k1 + e2 k2) at half steps e1, e2.  D2[k2][k1] samples the
+  // points of D2[k1][k2] with the mixed ones exchanged, and D2[k][k] the cell's
+  // own twice: 26 samples a cell in 3D for the 43 of the formula.
   for (int k1 = 0; k1 < dim; ++k1)
-    for (int k2 = 0; k2 < dim; ++k2) {
+    for (int k2 = k1; k2 < dim; ++k2) {
       float p00[3], p10[3], p01[3], p11[3];
       for (int a = 0; a < dim; ++a) {
         const float e1 = (a == k1) ? 0.5f : 0.0f, e2 = (a == k2) ? 0.5f : 0.0f;
@@ -638,9 +661,15 @@ __global__ void k_surface_b(Shape s, int d, Field u, Field phi, const float* __r
         p01[a] = (base - e1) + e2;
         p11[a] = (base + e1) + e2;
       }
-      float v00 = sample(u, p00), v10 = sample(u, p10), v01 = sample(u, p01),
-            v11 = sample(u, p11);
-      D2[k1][k2] = (((v11 + v00) - v10) - v01) / dx2;
+      const float v00 = sample(u, p00), v11 = sample(u, p11);
+      if (k1 == k2) {
+        if (k1 == 0) own = sample(u, p10);
+        D2[k1][k1] = (((v11 + v00) - own) - own) / dx2;
+      } else {
+        const float v10 = sample(u, p10), v01 = sample(u, p01);
+        D2[k1][k2] = (((v11 + v00) - v10) - v01) / dx2;
+        D2[k2][k1] = (((v11 + v00) - v01) - v10) / dx2;
+      }
     }
   float row[3];
   for (int j = 0; j < dim; ++j) {
@@ -915,8 +944,12 @@ extern "C" int mgpcg_potential_build_b(void* stream, int dim, const int32_t* res
   MG_REQUIRE(chi && H_ext && b, "NULL argument");
   for (int a = 0; a < dim; ++a) MG_REQUIRE(H_ext[a], "H_ext[%d] is NULL", a);
   Shape s = make_shape(dim, res);
-  hipLaunchKernelGGL(k_potential_b, dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream,
-                     s, Field{chi, s}, make_hfield(dim, res, H_ext), b);
+  if (dim == 3)
+    hipLaunchKernelGGL((k_potential_b<3>), dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream,
+                       s, Field{chi, s}, make_hfield(dim, res, H_ext), b);
+  else
+    hipLaunchKernelGGL((k_potential_b<2>), dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream,
+                       s, Field{chi, s}, make_hfield(dim, res, H_ext), b);
   MG_HIP(hipGetLastError());
   return 0;
 }
@@ -927,8 +960,12 @@ extern "C" int mgpcg_potential_build_A(void* stream, int dim, const int32_t* res
   MG_REQUIRE(chi && Adiag && Ax, "NULL argument");
   Shape s = make_shape(dim, res, level), fine = make_shape(dim, res);
   const float dxl = (float)(dx * (double)(1 << level));
-  hipLaunchKernelGGL(k_potential_A, dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream,
-                     s, fine, level, dxl, Field{chi, fine}, Adiag, Ax);
+  if (dim == 3)
+    hipLaunchKernelGGL((k_potential_A<3>), dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream,
+                       s, fine, level, dxl, Field{chi, fine}, Adiag, Ax);
+  else
+    hipLaunchKernelGGL((k_potential_A<2>), dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream,
+                       s, fine, level, dxl, Field{chi, fine}, Adiag, Ax);
   MG_HIP(hipGetLastError());
   return 0;
 }
@@ -943,8 +980,12 @@ extern "C" int mgpcg_surface_build_A(void* stream, int dim, const int32_t* res, 
   const float dxl = (float)(dx * (double)(1 << level));
   const float scale = (float)(sigma * dt) / (dxl * dxl);
   const float inv_dt = (float)(1.0 / dt);
-  hipLaunchKernelGGL(k_surface_A, dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream, s,
-                     fine, level, d, Field{phi, fine}, make_ls(dx), inv_dt, scale, Adiag, Ax);
+  if (dim == 3)
+    hipLaunchKernelGGL((k_surface_A<3>), dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream, s,
+                       fine, level, d, Field{phi, fine}, make_ls(dx), inv_dt, scale, Adiag, Ax);
+  else
+    hipLaunchKernelGGL((k_surface_A<2>), dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream, s,
+                       fine, level, d, Field{phi, fine}, make_ls(dx), inv_dt, scale, Adiag, Ax);
   MG_HIP(hipGetLastError());
   return 0;
 }
@@ -954,8 +995,12 @@ extern "C" int mgpcg_calc_n(void* stream, int dim, const int32_t* res, int d, co
   if (check_common(dim, res)) return -1;
   MG_REQUIRE(phi && n, "NULL argument");
   Shape s = make_shape(dim, res);
-  hipLaunchKernelGGL(k_calc_n, dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream, s, d,
-                     Field{phi, s}, (float)dx, n);
+  if (dim == 3)
+    hipLaunchKernelGGL((k_calc_n<3>), dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream, s, d,
+                       Field{phi, s}, (float)dx, n);
+  else
+    hipLaunchKernelGGL((k_calc_n<2>), dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream, s, d,
+                       Field{phi, s}, (float)dx, n);
   MG_HIP(hipGetLastError());
   return 0;
 }
@@ -965,8 +1010,12 @@ extern "C" int mgpcg_calc_kappa(void* stream, int dim, const int32_t* res, const
   if (check_common(dim, res)) return -1;
   MG_REQUIRE(n && kappa, "NULL argument");
   Shape s = make_shape(dim, res);
-  hipLaunchKernelGGL(k_calc_kappa, dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream, s,
-                     n, (float)dx, kappa);
+  if (dim == 3)
+    hipLaunchKernelGGL((k_calc_kappa<3>), dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream, s,
+                       n, (float)dx, kappa);
+  else
+    hipLaunchKernelGGL((k_calc_kappa<2>), dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream, s,
+                       n, (float)dx, kappa);
   MG_HIP(hipGetLastError());
   return 0;
 }
@@ -980,9 +1029,14 @@ extern "C" int mgpcg_surface_build_b(void* stream, int dim, const int32_t* res, 
   MG_REQUIRE(d >= 0 && d < dim, "axis d out of range");
   Shape s = make_shape(dim, res);
   Field u{velocity_d, make_shape(dim, res, 0, d)};
-  hipLaunchKernelGGL(k_surface_b, dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream, s,
-                     d, u, Field{phi, s}, kappa, n, make_ls(dx), (float)dt, (float)dx,
-                     (float)(dx * dx), (float)sigma, b);
+  if (dim == 3)
+    hipLaunchKernelGGL((k_surface_b<3>), dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream, s,
+                       d, u, Field{phi, s}, kappa, n, make_ls(dx), (float)dt, (float)dx,
+                       (float)(dx * dx), (float)sigma, b);
+  else
+    hipLaunchKernelGGL((k_surface_b<2>), dim3(nb_for(s.cells())), dim3(SB), 0, (hipStream_t)stream, s,
+                       d, u, Field{phi, s}, kappa, n, make_ls(dx), (float)dt, (float)dx,
+                       (float)(dx * dx), (float)sigma, b);
   MG_HIP(hipGetLastError());
   return 0;
 }
