@@ -124,6 +124,10 @@ int mgpcg_pool_bytes(int dim, const int32_t* res, int n_levels, int precision, i
  * full_reinitialize (mgpcg.py:79-94). */
 int mgpcg_load_level(mgpcg_solver_t* solver, int level, const int8_t* grid_type,
                      const float* Adiag, const float* Ax);
+/* mgpcg_load_level of every level and mgpcg_load_rhs at once, in two launches:
+ * grid_type[l], Adiag[l], Ax[l] for l < n_levels, and b. */
+int mgpcg_load(mgpcg_solver_t* solver, const int8_t* const* grid_type,
+               const float* const* Adiag, const float* const* Ax, const float* b);
 /* PressureProjectStrategy's reinitialize (pressure_project.py:15-64 via
  * mgpcg.py:79-87) straight into the device hierarchy: b and every level's
  * operator are computed in the packed layout, bit for bit what

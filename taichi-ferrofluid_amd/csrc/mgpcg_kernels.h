@@ -3287,7 +3287,47 @@ __global__ void __launch_bounds__(META_THREADS) k_meta_reduce(MetaReduceList ml)
   meta_reduce_level(ml, blockIdx.x);
 }
 
-// Packs one level from the canonical arrays (the strategies' output).
+// One slot (both colours) of a level packed from the canonical arrays (the
+// strategies' output); folds its coupling extremes and FLUID count into mn /
+// mx / wet / nfl.
+template <typename T, int DIM>
+__device__ __forceinline__ void pack_level_slot(const Geo& g, const int8_t* __restrict__ gt,
+                                                const float* __restrict__ Adiag,
+                                                const float* __restrict__ Ax,
+                                                const LevelPtrs<T>& P, int t, uint32_t& mn,
+                                                uint32_t& mx, uint32_t& wet, uint32_t& nfl) {
+  // every canonical value of both colours is loaded first (ghost slots and
+  // missing lower neighbours read cell 0 and discard it)
+  SlotCoefs<DIM> v[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const Slot sl = decode(g, t, c);
+    v[c].inn = sl.interior;
+    const long ci = sl.interior ? canon_index(g, sl.i, sl.j, sl.k) : 0;
+    const int x[3] = {sl.i, sl.j, sl.k};
+    long wi[DIM];
+#pragma unroll
+    for (int k = 0; k < DIM; ++k) {
+      // lower neighbour on original axis k (view axis k + 3 - DIM)
+      const int va = k + 3 - DIM;
+      v[c].hdn[k] = sl.interior && x[va] > 0;
+      int w[3] = {sl.i, sl.j, sl.k};
+      w[va] -= 1;
+      wi[k] = v[c].hdn[k] ? canon_index(g, w[0], w[1], w[2]) : 0;
+    }
+    v[c].gv = gt[ci];
+    v[c].ad = Adiag[ci];
+#pragma unroll
+    for (int k = 0; k < DIM; ++k) {
+      v[c].up[k] = Ax[ci * DIM + k];
+      v[c].dn[k] = Ax[wi[k] * DIM + k];
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 2; ++c) pack_slot<T, DIM>(v[c], c, t, P, mn, mx, wet, nfl);
+}
+
+// Packs one level.
 template <typename T, int DIM>
 __global__ void __launch_bounds__(BLOCK) k_pack_level(Geo g, const int8_t* __restrict__ gt,
                                                       const float* __restrict__ Adiag,
@@ -3295,37 +3335,7 @@ __global__ void __launch_bounds__(BLOCK) k_pack_level(Geo g, const int8_t* __res
                                                       LevelPtrs<T> P, uint32_t* part) {
   const int t = blockIdx.x * BLOCK + threadIdx.x;
   uint32_t mn = 0xffffffffu, mx = 0u, wet = 0u, nfl = 0u;
-  if (t < g.size) {
-    // every canonical value of both colours is loaded first (ghost slots and
-    // missing lower neighbours read cell 0 and discard it)
-    SlotCoefs<DIM> v[2];
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const Slot sl = decode(g, t, c);
-      v[c].inn = sl.interior;
-      const long ci = sl.interior ? canon_index(g, sl.i, sl.j, sl.k) : 0;
-      const int x[3] = {sl.i, sl.j, sl.k};
-      long wi[DIM];
-#pragma unroll
-      for (int k = 0; k < DIM; ++k) {
-        // lower neighbour on original axis k (view axis k + 3 - DIM)
-        const int va = k + 3 - DIM;
-        v[c].hdn[k] = sl.interior && x[va] > 0;
-        int w[3] = {sl.i, sl.j, sl.k};
-        w[va] -= 1;
-        wi[k] = v[c].hdn[k] ? canon_index(g, w[0], w[1], w[2]) : 0;
-      }
-      v[c].gv = gt[ci];
-      v[c].ad = Adiag[ci];
-#pragma unroll
-      for (int k = 0; k < DIM; ++k) {
-        v[c].up[k] = Ax[ci * DIM + k];
-        v[c].dn[k] = Ax[wi[k] * DIM + k];
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < 2; ++c) pack_slot<T, DIM>(v[c], c, t, P, mn, mx, wet, nfl);
-  }
+  if (t < g.size) pack_level_slot<T, DIM>(g, gt, Adiag, Ax, P, t, mn, mx, wet, nfl);
   pack_block_tail(mn, mx, wet, nfl, (uint8_t*)P.wet, (int32_t*)P.ord[0], part, blockIdx.x,
                   gridDim.x);
 }
@@ -3548,10 +3558,8 @@ __global__ void __launch_bounds__(BLOCK) k_pack_pressure_all(const PackLevel<T>*
 }
 
 template <typename S, typename D>
-__global__ void __launch_bounds__(BLOCK) k_pack_vec(Geo g, const S* __restrict__ src, D* d0,
-                                                    D* d1) {
-  const int t = blockIdx.x * BLOCK + threadIdx.x;
-  if (t >= g.size) return;
+__device__ __forceinline__ void pack_vec_slot(const Geo& g, const S* __restrict__ src, D* d0,
+                                              D* d1, int t) {
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
     Slot s = decode(g, t, c);
@@ -3559,6 +3567,40 @@ __global__ void __launch_bounds__(BLOCK) k_pack_vec(Geo g, const S* __restrict__
     if (s.interior) v = (D)src[canon_index(g, s.i, s.j, s.k)];
     (c ? d1 : d0)[t] = v;
   }
+}
+template <typename S, typename D>
+__global__ void __launch_bounds__(BLOCK) k_pack_vec(Geo g, const S* __restrict__ src, D* d0,
+                                                    D* d1) {
+  const int t = blockIdx.x * BLOCK + threadIdx.x;
+  if (t < g.size) pack_vec_slot<S, D>(g, src, d0, d1, t);
+}
+
+// Every level and b from the canonical arrays in one launch: a launch a level
+// kept the device to a few workgroups for most of them, and the host to two
+// launches each (2D 128^2, four levels: 57 us of kernels in ten launches).
+struct LoadCall {
+  const int8_t* gt[16];  // canonical arrays of each level
+  const float* Adiag[16];
+  const float* Ax[16];
+  int block0[17];
+  const float* b;
+  void* pb[2];  // level 0's packed b, both colours
+};
+template <typename T, int DIM>
+__global__ void __launch_bounds__(BLOCK) k_pack_all(const PackLevel<T>* __restrict__ tab,
+                                                    LoadCall c) {
+  int l = 0;
+  while ((int)blockIdx.x >= c.block0[l + 1]) ++l;
+  const PackLevel<T>& L = tab[l];
+  const int b = (int)blockIdx.x - c.block0[l];
+  const int t = b * BLOCK + threadIdx.x;
+  uint32_t mn = 0xffffffffu, mx = 0u, wet = 0u, nfl = 0u;
+  if (t < L.g.size) {
+    if (l == 0) pack_vec_slot<float, T>(L.g, c.b, (T*)c.pb[0], (T*)c.pb[1], t);
+    pack_level_slot<T, DIM>(L.g, c.gt[l], c.Adiag[l], c.Ax[l], L.P, t, mn, mx, wet, nfl);
+  }
+  pack_block_tail(mn, mx, wet, nfl, (uint8_t*)L.P.wet, (int32_t*)L.P.ord[0], L.part, b,
+                  c.block0[l + 1] - c.block0[l]);
 }
 
 template <typename S, typename D>

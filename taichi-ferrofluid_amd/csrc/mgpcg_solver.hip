@@ -1710,12 +1710,65 @@ extern "C" int mgpcg_load_rhs(mgpcg_solver_t* s, const float* b) {
 }
 
 namespace {
+// every level's record, and level 0's half-sweep order: one launch
+void finish_levels(mgpcg_solver* s) {
+  const int L = s->L;
+  MetaReduceList ml;
+  for (int l = 0; l < L; ++l) {
+    ml.meta[l] = s->lv[l].meta;
+    ml.part[l] = s->lv[l].part;
+    ml.nblocks[l] = nblk(s->geo[l].size);
+  }
+  const LevelBuf& B = s->lv[0];
+  const bool order = s->coarse_from > 0;
+  hipLaunchKernelGGL(k_finish_levels, dim3(L + (order ? 1 : 0)), dim3(META_THREADS), 0,
+                     s->user_stream, ml,
+                     L, B.wet, nblk(s->geo[0].size), order ? B.ord[1] : nullptr, B.ordtmp);
+}
+
+template <typename T>
+int load_t(mgpcg_solver* s, const int8_t* const* gt, const float* const* Adiag,
+           const float* const* Ax, const float* b) {
+  LoadCall c;
+  c.block0[0] = 0;
+  for (int l = 0; l < s->L; ++l) {
+    c.gt[l] = gt[l];
+    c.Adiag[l] = Adiag[l];
+    c.Ax[l] = Ax[l];
+    c.block0[l + 1] = c.block0[l] + nblk(s->geo[l].size);
+  }
+  c.b = b;
+  c.pb[0] = s->b[0];
+  c.pb[1] = s->b[1];
+  const PackLevel<T>* tab = (const PackLevel<T>*)s->packtab;
+  const dim3 grid(c.block0[s->L]), block(BLOCK);
+  if (s->dim == 3)
+    hipLaunchKernelGGL((k_pack_all<T, 3>), grid, block, 0, s->user_stream, tab, c);
+  else
+    hipLaunchKernelGGL((k_pack_all<T, 2>), grid, block, 0, s->user_stream, tab, c);
+  finish_levels(s);
+  MG_HIP(hipGetLastError());
+  return 0;
+}
+}  // namespace
+
+extern "C" int mgpcg_load(mgpcg_solver_t* s, const int8_t* const* grid_type,
+                          const float* const* Adiag, const float* const* Ax, const float* b) {
+  MG_REQUIRE(s != nullptr, "solver is NULL");
+  MG_REQUIRE(grid_type && Adiag && Ax && b, "NULL argument");
+  for (int l = 0; l < s->L; ++l)
+    MG_REQUIRE(grid_type[l] && Adiag[l] && Ax[l], "NULL field pointer (level %d)", l);
+  MG_HIP(hipSetDevice(s->device));
+  if (s->precision == F64) return load_t<double>(s, grid_type, Adiag, Ax, b);
+  return load_t<float>(s, grid_type, Adiag, Ax, b);
+}
+
+namespace {
 template <typename T>
 int assemble_pressure_t(mgpcg_solver* s, int8_t* const* gt, const float* const* velocity,
                         const float* phi, float sA, float sb, float p0, int gfm, float c_max,
                         int add_c, float cadd) {
   hipStream_t st = s->user_stream;
-  const Geo& g0 = s->geo[0];
   const int L = s->L;
   // the coarse levels' cell types, level by level (init_gridtype, mgpcg.py:46-60)
   for (int l = 1; l < L; ++l) {
@@ -1750,17 +1803,7 @@ int assemble_pressure_t(mgpcg_solver* s, int8_t* const* gt, const float* const* 
   else
     hipLaunchKernelGGL((k_pack_pressure_all<T, 2>), dim3(c.block0[L]), dim3(BLOCK), 0, st, tab,
                        c);
-  // every level's record, and level 0's half-sweep order: one launch
-  MetaReduceList ml;
-  for (int l = 0; l < L; ++l) {
-    ml.meta[l] = s->lv[l].meta;
-    ml.part[l] = s->lv[l].part;
-    ml.nblocks[l] = nblk(s->geo[l].size);
-  }
-  const LevelBuf& B = s->lv[0];
-  const bool order = s->coarse_from > 0;
-  hipLaunchKernelGGL(k_finish_levels, dim3(L + (order ? 1 : 0)), dim3(META_THREADS), 0, st, ml,
-                     L, B.wet, nblk(g0.size), order ? B.ord[1] : nullptr, B.ordtmp);
+  finish_levels(s);
   MG_HIP(hipGetLastError());
   return 0;
 }

@@ -55,6 +55,7 @@ SIGNATURES = {
     "mgpcg_pool_bytes": (_I, [_I, _P, _I, _I, _P]),
     "mgpcg_load_level": (_I, [_P, _I, _P, _P, _P]),
     "mgpcg_load_rhs": (_I, [_P, _P]),
+    "mgpcg_load": (_I, [_P, _P, _P, _P, _P]),
     "mgpcg_level_coupling": (_I, [_P, _I, ctypes.POINTER(_I), ctypes.POINTER(ctypes.c_float)]),
     "mgpcg_level_flags": (_I, [_P, _I, _P, _P]),
     "mgpcg_level_order": (_I, [_P, _I, _P, _P]),

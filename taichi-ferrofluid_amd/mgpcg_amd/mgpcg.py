@@ -171,10 +171,11 @@ class MGPCGPoissonSolver:
             return
         h = self._h
         _lib.check(self._lib.mgpcg_set_stream(h, _lib.stream_handle(self.device)))
-        for l in range(self.n_mg_levels):
-            _lib.check(self._lib.mgpcg_load_level(h, l, _lib.ptr(self.grid_type[l]),
-                                                  _lib.ptr(self.Adiag[l]), _lib.ptr(self.Ax[l])))
-        _lib.check(self._lib.mgpcg_load_rhs(h, _lib.ptr(self.b)))
+        for t in [self.b, *self.grid_type, *self.Adiag, *self.Ax]:
+            _lib.ptr(t)  # what it refuses stays refused
+        _lib.check(self._lib.mgpcg_load(h, _lib.ptr_array(self.grid_type),
+                                        _lib.ptr_array(self.Adiag), _lib.ptr_array(self.Ax),
+                                        _lib.ptr(self.b)))
 
     # -- solve -------------------------------------------------------------------
     def solve(self, max_iters=-1, verbose=False, rel_tol=1e-12, abs_tol=1e-14, eps=1e-12):
