@@ -262,7 +262,9 @@ int mgpcg_graph_counts(const mgpcg_solver_t* solver, const mgpcg_batch_t* batch,
 
 /* Kernel-level access for parity tests (no reference counterpart): move a
  * level vector between canonical layout (float, or double for MGPCG_F64 and
- * for x outside MGPCG_PLAIN) and the handle, and run one stage. */
+ * for x outside MGPCG_PLAIN) and the handle, and run one stage.  R and Z of a
+ * level are what mgpcg_debug_op left; a solve keeps them in memory only as far
+ * as its kernels read them there (not below the coarse kernel's first level). */
 #define MGPCG_FIELD_R 0
 #define MGPCG_FIELD_Z 1
 #define MGPCG_FIELD_P 2      /* p buffer of even iterations */

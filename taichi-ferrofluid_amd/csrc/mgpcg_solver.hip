@@ -252,6 +252,7 @@ struct Engine {
   StageRef st_init, st_cg, fin_init, fin_cg, fin_all, st_dot_fused, st_dot_plain, st_coarse,
       st_gather;
   bool coarse_lds = false;  // every coarse item's levels fit the coarse kernel's LDS image
+  bool keep_levels = false;  // ... which also leaves every level's z and r in memory
   int restrict_mode = 0;    // restriction stages of level 0 are laid out for this mode
   int restrict_mode_c = 0;  // ... and those of the levels below it for this one
   std::vector<StageRef> st_slot, st_restrict, st_bottom;  // per level
@@ -908,12 +909,12 @@ struct Sched {
           hipLaunchKernelGGL((k_coarse<T, DIM, true>), dim3(e->st_coarse.n),
                              dim3(COARSE_THREADS), 0, e->stream, levels(e),
                              (const Item*)(e->d_items + e->st_coarse.off), e->st_coarse.n,
-                             e->st_coarse.one, nu, e->bottom);
+                             e->st_coarse.one, nu, e->bottom, e->keep_levels);
       }
       if (!lds)
         hipLaunchKernelGGL((k_coarse<T, DIM, false>), dim3(e->st_coarse.n), dim3(COARSE_THREADS),
                            0, e->stream, levels(e), (const Item*)(e->d_items + e->st_coarse.off),
-                           e->st_coarse.n, e->st_coarse.one, nu, e->bottom);
+                           e->st_coarse.n, e->st_coarse.one, nu, e->bottom, true);
     }
     for (int l = L - 2; l >= 0; --l) {
       if (tiled(e, l)) {
@@ -2180,7 +2181,9 @@ extern "C" int mgpcg_debug_op(mgpcg_solver_t* s, int op, int level, int arg) {
   if (engine_build_items(e)) return -2;
   MG_HIP(hipStreamSynchronize(e->stream));
   if (op == MGPCG_OP_VCYCLE) {
+    e->keep_levels = true;
     dispatch<RunVcycle>(e->precision, e->dim, e);
+    e->keep_levels = false;
   } else {
     Engine::StageRef r;
     if (prepare_op(e, s, op, level, &r)) return -2;
