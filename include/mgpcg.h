@@ -369,8 +369,9 @@ int mgpcg_apply_markers(void* stream, int dim, const int32_t* res, const float* 
 int mgpcg_init_boundary(void* stream, int dim, const int32_t* res, int8_t* cell_type);
 /* FastSweepingLevelSet.redistance (level_set.py:260-333), phi in place;
  * phi_temp, snap (floats) and fixed (bytes) are caller-provided work arrays
- * of the grid's size.  Neighbouring lines are read as they were before each
- * sweep (deterministic; the reference's parallel lines race). */
+ * of the grid's size; phi_temp is left with the new distances too.
+ * Neighbouring lines are read as they were before each sweep (deterministic;
+ * the reference's parallel lines race). */
 int mgpcg_redistance(void* stream, int dim, const int32_t* res, double dx, int repeat_times,
                      float* phi, float* phi_temp, float* snap, int8_t* fixed);
 

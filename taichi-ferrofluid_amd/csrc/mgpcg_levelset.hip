@@ -21,6 +21,7 @@
 #include <math.h>
 
 #include <type_traits>
+#include <utility>
 
 #include "../../include/mgpcg.h"
 #include "mgpcg_common.h"
@@ -219,10 +220,13 @@ constexpr int SW_FILL = 256;
 constexpr int SW_THREADS = 64 + SW_FILL;
 constexpr int SW_MINE = SW_LINES * SW_STEPS / SW_FILL;  // places per filling thread
 constexpr int SW_WORDS = SW_LINES * (SW_STEPS + 1);     // one step more: the chunk's next cell
+// also: NULL, or (on axis 0, in the last sweep) a second array for the
+// distances, which a copy after it would read again.
 template <int DIM, int AX, bool ROOT, typename IX>
 __global__ void __launch_bounds__(SW_THREADS, 5) k_sweep(Grid g, int dir,
                                                       const float* __restrict__ src,
                                                       float* __restrict__ dst,
+                                                      float* __restrict__ also,
                                                       const int8_t* __restrict__ code,
                                                       EikonalConsts c) {
   constexpr bool CONTIG = AX == DIM - 1;
@@ -291,6 +295,10 @@ __global__ void __launch_bounds__(SW_THREADS, 5) k_sweep(Grid g, int dir,
       const IX t = first[CONTIG ? i : 0] + s * st;
       if constexpr (sizeof(IX) == 4) stgi(dst, t, v);
       else stg(dst + t, v);
+      if (AX == 0 && also != nullptr) {
+        if constexpr (sizeof(IX) == 4) stgi(also, t, v);
+        else stg(also + t, v);
+      }
     }
   };
   auto store = [&](int chunk) {
@@ -625,7 +633,7 @@ __global__ void __launch_bounds__(LB, 6) k_diffuse(Faces3 F, int from) {
 inline unsigned nblk(long n) { return (unsigned)((n + LB - 1) / LB); }
 
 template <int DIM, int AX>
-void sweep_t(hipStream_t s, const Grid& g, int dir, const float* src, float* dst,
+void sweep_t(hipStream_t s, const Grid& g, int dir, const float* src, float* dst, float* also,
              const int8_t* code, const EikonalConsts& c) {
   const long nlines = g.cells() / g.n[AX];
   const dim3 grid((unsigned)((nlines + SW_LINES - 1) / SW_LINES));
@@ -634,26 +642,26 @@ void sweep_t(hipStream_t s, const Grid& g, int dir, const float* src, float* dst
   // 2^-96 for every dx but the smallest.  32-bit offsets reach 2^30 cells.
   if (c.dx < 0x1p-32f)
     hipLaunchKernelGGL((k_sweep<DIM, AX, false, long>), grid, dim3(SW_THREADS), 0, s, g, dir, src,
-                       dst, code, c);
+                       dst, also, code, c);
   else if (g.cells() > (1l << 30))
     hipLaunchKernelGGL((k_sweep<DIM, AX, true, long>), grid, dim3(SW_THREADS), 0, s, g, dir, src,
-                       dst, code, c);
+                       dst, also, code, c);
   else
     hipLaunchKernelGGL((k_sweep<DIM, AX, true, int>), grid, dim3(SW_THREADS), 0, s, g, dir, src,
-                       dst, code, c);
+                       dst, also, code, c);
 }
 
 void sweep(hipStream_t s, const Grid& g, int ax, int dir, const float* src, float* dst,
-           const int8_t* code, const EikonalConsts& c) {
+           float* also, const int8_t* code, const EikonalConsts& c) {
   if (g.dim == 2) {
-    if (ax == 0) sweep_t<2, 0>(s, g, dir, src, dst, code, c);
-    else sweep_t<2, 1>(s, g, dir, src, dst, code, c);
+    if (ax == 0) sweep_t<2, 0>(s, g, dir, src, dst, also, code, c);
+    else sweep_t<2, 1>(s, g, dir, src, dst, also, code, c);
   } else if (ax == 0) {
-    sweep_t<3, 0>(s, g, dir, src, dst, code, c);
+    sweep_t<3, 0>(s, g, dir, src, dst, also, code, c);
   } else if (ax == 1) {
-    sweep_t<3, 1>(s, g, dir, src, dst, code, c);
+    sweep_t<3, 1>(s, g, dir, src, dst, also, code, c);
   } else {
-    sweep_t<3, 2>(s, g, dir, src, dst, code, c);
+    sweep_t<3, 2>(s, g, dir, src, dst, also, code, c);
   }
 }
 
@@ -711,16 +719,16 @@ extern "C" int mgpcg_redistance(void* stream, int dim, const int32_t* res, doubl
     hipLaunchKernelGGL((k_target_surface<2>), dim3(nblk(n)), dim3(LB), 0, s, g,
                        (const float*)phi, (float)dx, phi_temp, fixed);
   // each sweep reads one work array and writes the other; the last one writes
-  // phi, which nothing reads after target_surface
-  const float* src = phi_temp;
-  float* dst = snap;
+  // phi, which nothing reads after target_surface, and phi_temp, which it does
+  // not read (an even number of sweeps: the one before it wrote snap)
+  float *src = phi_temp, *dst = snap;
   for (int rep = 0; rep < repeat_times; ++rep) {
     for (int ax = dim - 1; ax >= 0; --ax) {
       for (int dir = 1; dir >= -1; dir -= 2) {
-        float* out = rep == repeat_times - 1 && ax == 0 && dir == -1 ? phi : dst;
-        sweep(s, g, ax, dir, src, out, (const int8_t*)fixed, c);
-        dst = const_cast<float*>(src);
-        src = out;
+        const bool last = rep == repeat_times - 1 && ax == 0 && dir == -1;
+        sweep(s, g, ax, dir, src, last ? phi : dst, last ? dst : nullptr, (const int8_t*)fixed,
+              c);
+        std::swap(src, dst);
       }
     }
   }

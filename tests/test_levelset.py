@@ -126,3 +126,19 @@ def test_redistance_at_tile_edges(dev, res):
     with np.errstate(all="ignore"):
         ref = OL.redistance(phi, dx, 2)
     assert np.array_equal(ls.phi.cpu().numpy(), ref, equal_nan=True)
+
+
+@pytest.mark.parametrize("repeat", [0, 1, 2])
+@pytest.mark.parametrize("res", [(24, 20), (65, 17), (14, 12, 16), (5, 13, 31)],
+                         ids=lambda r: "x".join(map(str, r)))
+def test_redistance_leaves_the_distances_in_phi_temp_too(dev, res, repeat):
+    from mgpcg_amd.level_set import FastSweepingLevelSet
+
+    # a small ball at the far end of axis 0: the last sweep reaches most cells
+    phi = _sphere(res, [0.37 * (n - 1.9) for n in res], 0.5, 0.37).astype(np.float32)
+    ls = FastSweepingLevelSet(len(res), res, 0.37, phi=_t(phi, dev), device=dev)
+    ls.repeat_times = repeat
+    ls.redistance()
+    ref = OL.redistance(phi, 0.37, repeat)
+    assert np.array_equal(ls.phi.cpu().numpy(), ref)
+    assert np.array_equal(ls.phi_temp.cpu().numpy(), ref)
