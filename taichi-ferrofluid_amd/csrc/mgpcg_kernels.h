@@ -1067,8 +1067,13 @@ enum StageOp {
 // coarser levels, 1 level 0, 2 level 0's smooth(0) launches that the launch
 // probe records (so a profiler's statistics of that instantiation cover
 // exactly the launches the probe timed).
+// At most 80 SGPRs: a SIMD holds 800, a wave takes its own in sixteens and 16
+// more for the trap handler, so a kernel with more than 80 has 7 waves per SIMD
+// and not 8, and the workgroups of a full persistent launch are not all
+// resident.  With 84 the probed launches took 21.2 us where the same code
+// without the probe takes 16.8 (one 256^3 system), and 43 for 34 (two).
 template <typename T, int DIM, int OP, int L0>
-__global__ void __launch_bounds__(BLOCK) k_stage(const LevelDesc<T>* __restrict__ descs,
+__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_num_sgpr(80))) k_stage(const LevelDesc<T>* __restrict__ descs,
                                                  Stage S) {
   ItemCache ic;
   bool done = true;
