@@ -101,9 +101,10 @@ int mgpcg_set_stream(mgpcg_solver_t* solver, void* stream);
                                         modes of MGPCG_OPT_RESTRICT_ROWS; -1 (default): the
                                         MGPCG_OPT_RESTRICT_ROWS mode */
 /* A level whose members take at most this many blocks of 8^3 cells together
- * (in 2D four times as many, of 24^2) runs its pre-smoothing with the
- * restriction, and its prolongation with the post-smoothing, in one launch
- * each (default 768, 0: never). */
+ * (two thirds of it in FP64; in 2D four times as many, of 24^2) runs its
+ * pre-smoothing with the restriction, and its prolongation with the
+ * post-smoothing, in one launch each (default 768, 0: never), with two
+ * smoothing steps, in 2D also with one. */
 enum { MGPCG_OPT_TILE_MAX = 16 };
 int mgpcg_set_option(mgpcg_solver_t* solver, int option, int value);
 /* The current value of a knob (no reference counterpart; `solver` is unused). */

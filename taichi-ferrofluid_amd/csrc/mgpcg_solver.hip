@@ -837,10 +837,20 @@ struct Sched {
   // Measured, half-sweeps against legs, whole solves: level 1 of 72x48x88
   // (594 blocks) 4.71 -> 4.46 ms; of 88x80x72, all FLUID (990) 54.9 -> 60.2 ms;
   // level 0 of 96x112x88 (1848) 2.65 -> 3.48 ms.  A 2D block has a quarter of
-  // the cells and little overlap: 1024^2 (1849 blocks) 3.75 -> 3.37 ms.
+  // the cells and little overlap: 1024^2 (1849 blocks) 3.75 -> 3.37 ms, 1296^2
+  // (2916) 5.68 -> 3.85, in FP64 8.94 -> 6.21.
+  // With one smoothing step the legs save two launches a level less and their
+  // layers are as deep: all FLUID, half-sweeps against legs, 40^3 (125 blocks)
+  // 2.06 -> 2.56 ms, 64^3 (512) 2.34 -> 2.85, so 3D has them with two only; in 2D
+  // they win, 256^2 2.32 -> 1.96.
+  // FP64 doubles a block's LDS traffic, and its divisions cost four times as
+  // much: all FLUID, 64^3 (512) 5.07 -> 4.82 ms, 64x64x80 (640) 5.44 -> 5.70, 72x64x80 (720)
+  // 5.83 -> 6.33, so it has two blocks per CU, where FP32 has three.
   static bool tiled(const Engine* e, int l) {
-    const long n = e->st_tile[l].nblocks, most = (DIM == 3 ? 1l : 4l) * g_tile_max;
-    return n > 0 && n <= most && e->nu >= 1 && e->nu <= TILE_MAX_NU &&
+    const long n = e->st_tile[l].nblocks,
+               most = DIM == 2 ? 4l * g_tile_max
+                               : (sizeof(T) == 4 ? 1l * g_tile_max : 2l * g_tile_max / 3);
+    return n > 0 && n <= most && e->nu >= (DIM == 2 ? 1 : TILE_MAX_NU) && e->nu <= TILE_MAX_NU &&
            g_fuse_first == 0 && g_fuse_prolong && restrict_mode_of(e, l) == 2 &&
            !(l == 0 && e->probe_on);  // the probe times level 0's half-sweeps
   }

@@ -159,7 +159,9 @@ unsigned long long ballot(int pred) {
   return m;
 }
 
+long g_launches = 0;  // kernels run so far
 void run_grid(dim3 grid, dim3 block, void (*tramp)(void*), void* ctx) {
+  ++g_launches;
   gridDim = grid;
   blockDim = block;
   g_tramp = tramp;
@@ -299,6 +301,9 @@ void submit(hipStream_t s, std::function<void()> op) {
     op();
 }
 }  // namespace hipemu
+
+// kernels run so far
+extern "C" long hipemu_launches(void) { return hipemu::g_launches; }
 
 // operations queued on the library's streams (deferred streams only)
 extern "C" long hipemu_queued(void) {

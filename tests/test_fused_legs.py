@@ -32,3 +32,32 @@ def test_fused_legs_are_the_half_sweeps(dev, res, L, nu, kind, precision):
         _lib.check(lib.mgpcg_set_option(None, _lib.OPT_COARSE_MAX_SLOTS, 4096))
     assert out[0][1]["iters"] == out[1][1]["iters"]
     assert np.array_equal(out[0][0], out[1][0])
+
+
+# the FP32 limit is 768 blocks in 3D, the FP64 one 512, the 2D one 3072
+@pytest.mark.parametrize("res,nu,precision,limit,legs", [
+    ([16, 16, 16], 2, "plain", 8, True), ([16, 16, 16], 2, "plain", 7, False),
+    ([16, 16, 16], 1, "plain", 768, False), ([16, 16, 16], 1, "f64", 768, False),
+    ([16, 24, 16], 2, "f64", 18, True), ([16, 24, 16], 2, "f64", 17, False),
+    ([48, 48], 2, "plain", 1, True), ([48, 72], 2, "f64", 1, False),
+    ([48, 48], 1, "mixed", 1, True), ([48, 48], 1, "f64", 1, True)])
+def test_where_the_fused_legs_run(dev, res, nu, precision, limit, legs):
+    """The rule on blocks, smoothing steps and type, by the launches of a solve."""
+    from mgpcg_amd import _lib
+
+    lib = _lib.load()
+    if not hasattr(lib, "hipemu_launches"):
+        pytest.skip("counts the emulator's launches")
+    sysd = dict(scenes.pool_sphere_system(res, 7, L=2, kind="psi"), nu=nu)
+    count = []
+    try:
+        _lib.check(lib.mgpcg_set_option(None, _lib.OPT_COARSE_MAX_SLOTS, 0))
+        for blocks in (0, limit):
+            _lib.check(lib.mgpcg_set_option(None, _lib.OPT_TILE_MAX, blocks))
+            n = lib.hipemu_launches()
+            gpu_solve(sysd, dev, precision, max_iters=1)
+            count.append(lib.hipemu_launches() - n)
+    finally:
+        _lib.check(lib.mgpcg_set_option(None, _lib.OPT_TILE_MAX, 768))
+        _lib.check(lib.mgpcg_set_option(None, _lib.OPT_COARSE_MAX_SLOTS, 4096))
+    assert (count[1] < count[0]) == legs and (count[1] == count[0]) != legs
