@@ -1934,14 +1934,20 @@ __device__ void coarse_bottom(const Geo& g, const LevelPtrs<T>& P, int bottom) {
 // a batch's 16 systems, 39 us now).  Solves: 128^3 4.32 -> 3.95 ms, 128^2
 // 857 -> 790 us, batch of 16 97 -> 75 ms.
 //
-// The first coarse level has at most CZ_MAX_SLOTS slots per colour; with its
-// ghost layers off, at most 3 cells per lane and colour in 3D
-// ((n0 + 2)(n1 + 2)(n2 + 3) / 2 <= 4096 gives n0 n1 n2 / 2 < 2830) and 4 in 2D.
-// The levels below have a fourth of its cells or fewer: one per lane.
+// The first coarse level has at most CZ_MAX_SLOTS slots per colour, (n0 + 2)
+// (n1 + 2) times (n2 + 3) / 2 rounded down; with its ghost layers off, at most 3
+// cells per lane and colour in 3D (15 x 22 x 18 has the most of any shape, 2970)
+// and 4 in 2D (89 x 88: 3916).  The levels below have a fourth of its cells or
+// fewer (977 per colour): one per lane.  The host checks both (cz_fits).
 constexpr int CZ_MAX_SLOTS = 4096;
 template <int DIM>
 __host__ __device__ constexpr int cz_slots() {
   return DIM == 3 ? 3 : 4;
+}
+// Whether a level's lists fit the lanes' rows (first: the first coarse level).
+inline bool cz_fits(const Geo& g, bool first) {
+  const int rows = !first ? 1 : (g.dim == 3 ? cz_slots<3>() : cz_slots<2>());
+  return g.size <= CZ_MAX_SLOTS && (g.ncells + 1) / 2 <= rows * COARSE_THREADS;
 }
 constexpr int COARSE_LDS_BYTES = 160 * 1024 - 256;  // the rest: the lists' lengths
 constexpr int CZ_MAX_LEVELS = 16;

@@ -685,13 +685,15 @@ int engine_build_items(Engine* e) {
     x.desc = m * L + M.s->coarse_from;
     x.block0 = L - M.s->coarse_from;
     it.push_back(x);
-    if (M.s->geo[M.s->coarse_from].size > CZ_MAX_SLOTS) {
-      e->coarse_lds = false;
-      continue;
-    }
     long bytes = 0;
-    for (int l = M.s->coarse_from; l < L; ++l)
-      bytes += coarse_image_bytes(M.s->geo[l].size, (int)M.s->esz);
+    for (int l = M.s->coarse_from; l < L; ++l) {
+      const Geo& g = M.s->geo[l];
+      if (!cz_fits(g, l == M.s->coarse_from)) {
+        e->coarse_lds = false;
+        break;
+      }
+      bytes += coarse_image_bytes(g.size, (int)M.s->esz);
+    }
     if (bytes > COARSE_LDS_BYTES) e->coarse_lds = false;
   }
   e->st_coarse.n = (int)it.size() - e->st_coarse.off;

@@ -63,3 +63,23 @@ def test_lds_coarse_levels_leave_every_levels_fields(dev, res, L, p_air):
         cells = (h["gt"][i % L] == 0) | (i >= L)
         assert np.array_equal(a[cells], b[cells]), (("z", "r")[i // L], i % L)
     assert p_air > 0.0 or all((g == 0).any() for g in h["gt"])
+
+
+@pytest.mark.parametrize("res,L", [([18, 18, 18], 2), ([15, 22, 18], 1), ([89, 88], 1)])
+def test_lds_coarse_levels_with_the_most_cells(dev, res, L):
+    """The shapes of up to 4096 slots per colour with the most cells, all FLUID:
+    2916 and 2970 per colour in 3D, 3916 in 2D."""
+    from mgpcg_amd import _lib
+
+    print(f"case {res} L={L} on {dev}", flush=True)
+    sysd = scenes.pool_sphere_system(res, 3, L=L, kind="psi")
+    lib = _lib.load()
+    out = []
+    try:
+        for lds in (0, 1):
+            _lib.check(lib.mgpcg_set_option(None, _lib.OPT_COARSE_LDS, lds))
+            out.append(gpu_solve(sysd, dev, "plain", max_iters=3))
+    finally:
+        _lib.check(lib.mgpcg_set_option(None, _lib.OPT_COARSE_LDS, 1))
+    assert out[0][1]["iters"] == out[1][1]["iters"]
+    assert np.array_equal(out[0][0], out[1][0])
