@@ -142,3 +142,21 @@ def test_redistance_leaves_the_distances_in_phi_temp_too(dev, res, repeat):
     ref = OL.redistance(phi, 0.37, repeat)
     assert np.array_equal(ls.phi.cpu().numpy(), ref)
     assert np.array_equal(ls.phi_temp.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("dx", [0.37, 2.0 ** -32, 0.99 * 2.0 ** -32, 1e-10],
+                         ids=["0.37", "2^-32", "below", "1e-10"])
+@pytest.mark.parametrize("res", [(65, 17), (64, 15), (7, 9, 16), (5, 13, 31), (17, 3, 33)],
+                         ids=lambda r: "x".join(map(str, r)))
+def test_redistance_on_both_sides_of_the_smallest_dx(dev, res, dx):
+    """From dx = 2^-32 down the sweeps take the general square root and 64-bit
+    offsets: bit for bit on either side of it."""
+    from mgpcg_amd.level_set import FastSweepingLevelSet
+
+    rng = np.random.default_rng(list(res))
+    d = _sphere(res, [0.3 * n for n in res], 0.31 * min(res) + 0.2, 1.0)
+    phi = (dx * d * rng.uniform(0.5, 3.0, res)).astype(np.float32)
+    phi[rng.uniform(size=res) < 0.02] = 0.0
+    ls = FastSweepingLevelSet(len(res), res, dx, phi=_t(phi, dev), device=dev)
+    ls.redistance()
+    assert np.array_equal(ls.phi.cpu().numpy(), OL.redistance(phi, dx, 2))
