@@ -881,9 +881,7 @@ __device__ __forceinline__ int parent_slot(const Geo& gf, const Geo& gc, int t, 
 // ---------------------------------------------------------------------------
 // per-slot stage bodies (shared by the batched kernels and the coarse kernel)
 // ---------------------------------------------------------------------------
-// The slot bodies take the level's z colour arrays explicitly (z[0], z[1]):
-// the batched kernels pass the level's own arrays, the coarse kernel copies
-// held in LDS.
+// The slot bodies take the level's z colour arrays explicitly (z[0], z[1]).
 
 // smooth(l, c) (mgpcg.py:104-109) at slot t of colour c.
 template <typename T, int DIM>
@@ -1379,9 +1377,9 @@ __global__ void __launch_bounds__(BLOCK) k_restrict_gather(const LevelDesc<T>* _
 // of them wet) where its launches took 27 and 30 us (before) and 19 and 22 us
 // (after); 6 us on a 128^2 level 0 for 21 us.  What is left is the launch, the
 // two dependent reads before the first operand, and VALU issue: 38 instructions
-// per slot update, the exact division 10 of them.  80 VGPRs leave one 3D
-// workgroup per CU; asked for two (64 VGPRs, 14 spilled) a 128^3 solve went
-// from 4.32 to 4.55 ms.  Whole solves: 128^2 1055 -> 857 us, 128^3 5.33 ->
+// per slot update, the exact division 10 of them.  80 VGPRs (118 in level 0's
+// second leg, which forms z.r) leave one 3D workgroup per CU; asked for two
+// (64 VGPRs, 14 spilled) a 128^3 solve went from 4.32 to 4.55 ms.  Whole solves: 128^2 1055 -> 857 us, 128^3 5.33 ->
 // 4.35 ms, 256^3 20.5 -> 19.2 ms.
 constexpr int TILE_HALO = 4;      // deepest dependency chain of a leg that fits
 constexpr int TILE_MAX_NU = 2;    // smoothing steps: 2 * nu half-sweeps <= TILE_HALO
@@ -1924,8 +1922,10 @@ __device__ void coarse_bottom(const Geo& g, const LevelPtrs<T>& P, int bottom) {
 // FLUID slots for the whole V-cycle: the FLUID slots of each level and colour
 // are listed once (ghost, AIR and SOLID slots cost nothing afterwards), and a
 // lane keeps each of its slots' right-hand side, couplings, diagonal and
-// reciprocal diagonal in registers; LDS holds z and the residuals.  Levels
-// with stored couplings (potential, surface tension) run the same phases.
+// reciprocal diagonal to itself, in registers but for 21 (2D: 15) of them that
+// the 128 of a 1024-lane workgroup do not hold and that go to scratch memory;
+// LDS holds z and the residuals.  Levels with stored couplings (potential,
+// surface tension) run the same phases.
 // The arithmetic is the global-memory form's, operation for operation.
 // Before, every phase decoded and re-read each slot of an LDS image of the
 // whole level: 32.8 -> 19.0 us a V-cycle at 128^3 (levels of 16^3 and 8^3
@@ -2222,7 +2222,7 @@ __device__ void cz_vcycle(const LevelDesc<T>* descs, int d0, int nlev, int nu, i
     for (int j = 0; j < k; ++j) o += coarse_image_bytes(descs[d0 + j].g.size, (int)sizeof(T));
     return o;
   };
-  // the first two levels' rows stay in registers; the levels below (and only
+  // the first two levels' rows are held throughout; the levels below (and only
   // they) load theirs at each visit
   const Geo gA = descs[d0].g;
   const LevelPtrs<T> PA = descs[d0].P;
@@ -2402,9 +2402,10 @@ __device__ __forceinline__ void first_z0(const LevelPtrs<T>& P, const Coupling<T
 }
 
 // ---------------------------------------------------------------------------
-// CG kernels on level 0 (mgpcg.py:150-238).  Reductions: one double-double
-// partial per virtual block (a workgroup run's total in its first virtual
-// block, zero in the others); a per-system finalize kernel sums them.
+// CG kernels on level 0 (mgpcg.py:150-238).  Reductions: a workgroup leaves one
+// double-double per system, in the entry of its first virtual block there (the
+// other entries hold what an earlier launch left); a per-system finalize kernel
+// sums those that run_first names.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ double rnd_plain(const CGState* st, double v) {
   return st->precision == PLAIN ? (double)(float)v : v;
