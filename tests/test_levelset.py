@@ -111,7 +111,8 @@ def test_redistance_matches_oracle(dev, res, repeat):
                                  (3, 65, 15)], ids=lambda r: "x".join(map(str, r)))
 def test_redistance_at_tile_edges(dev, res):
     """Lines and chunks that end inside, at and just past a tile of the sweep
-    kernels (64 lines, 16 steps), with infinities and repeated zeros in the level set: bit for bit."""
+    kernels (64 lines, 16 steps), with infinities and repeated zeros in the
+    level set: bit for bit."""
     from mgpcg_amd.level_set import FastSweepingLevelSet
 
     rng = np.random.default_rng(list(res))
