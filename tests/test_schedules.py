@@ -71,3 +71,26 @@ def test_batch_of_different_first_levels_equals_alone(dev, tile_max, max_grid):
         xa, ra, _ = gpu_solve(sysd, dev, "mixed", max_iters=4)
         assert ra["iters"] == rb["iters"] and ra["rr"] == rb["rr"]
         assert np.array_equal(xa, xb)
+
+
+# level 0 in blocks of 256 slots: fewer than the eight groups of a launch, as
+# many, a multiple of them and others
+@pytest.mark.parametrize("L", [1, 2])
+@pytest.mark.parametrize("res,blocks", [([14, 28], 1), ([30, 24], 2), ([62, 50], 7), ([62, 60], 8),
+                                        ([62, 66], 9), ([62, 124], 16), ([62, 130], 17),
+                                        ([94, 124], 24), ([94, 130], 25)])
+def test_dot_products_at_block_counts(dev, res, blocks, L):
+    """Finalize sums the partial of every workgroup and no other entry, whatever
+    the launch's shape; with two levels the launches of z.r (the legs' blocks of
+    24^2) and of the other products leave theirs in different entries."""
+    sysd = scenes.pool_sphere_system(res, 9, L=L, kind="pressure")
+    slots = (res[0] + 2) * ((res[1] + 3) // 2)
+    assert (slots + 255) // 256 == blocks
+    set_knobs(coarse_max=0)
+    try:
+        x, out, _ = gpu_solve(sysd, dev, "plain", max_iters=4)
+    finally:
+        set_knobs(**KNOB_DEFAULTS)
+    xr, outr, _ = osys.solve(sysd, core.PLAIN, max_iters=4, rel_tol=1e-12)
+    assert out["iters"] == outr["iters"]
+    assert np.array_equal(x, xr)
