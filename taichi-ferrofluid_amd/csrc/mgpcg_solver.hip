@@ -76,6 +76,16 @@ constexpr int MAX_LANES = 4;  // most engines per server (the lane stream pool's
 int g_graph = 0;          // replay iterations of an unchanged member set from a hipGraph
 long g_knob_epoch = 0;    // bumped by every option change (captured graphs go stale)
 
+// The options that several launches of one iteration have to agree on (a
+// level's two legs, a launch and the finalize that reads its partials): read
+// once as it begins, whatever another thread sets meanwhile.
+struct Knobs {
+  int max_grid, tile_max, fuse_first, fuse_prolong, fuse_p;
+};
+Knobs knobs_now() {
+  return {g_max_grid, g_tile_max, g_fuse_first, g_fuse_prolong, g_fuse_p};
+}
+
 }  // namespace
 
 struct Engine;
@@ -251,6 +261,7 @@ struct Engine {
   };
   StageRef st_init, st_cg, fin_init, fin_cg, fin_all, st_dot_fused, st_dot_plain, st_coarse,
       st_gather;
+  Knobs kn = knobs_now();   // of the iteration being enqueued
   bool coarse_lds = false;  // every coarse item's levels fit the coarse kernel's LDS image
   bool keep_levels = false;  // ... which also leaves every level's z and r in memory
   int restrict_mode = 0;    // restriction stages of level 0 are laid out for this mode
@@ -766,8 +777,9 @@ inline Stage stage_of(const Engine* e, const Engine::StageRef& r) {
   s.t1 = nullptr;
   return s;
 }
-inline int grid_of(const Engine::StageRef& r) { return std::min(r.nblocks, g_max_grid); }
-
+inline int grid_of(const Engine* e, const Engine::StageRef& r) {
+  return std::min(r.nblocks, e->kn.max_grid);
+}
 
 // ---------------------------------------------------------------------------
 // iteration schedule, templated on hierarchy type T, x type TX and dimension
@@ -787,13 +799,13 @@ struct Sched {
         st.swept = e->d_swept;
         st.t0 = e->d_span + (size_t)e->probe_used * SPAN_SLOTS;
         st.t1 = e->d_span + (size_t)(PROBE_POOL + e->probe_used) * SPAN_SLOTS;
-        hipLaunchKernelGGL((k_stage<T, DIM, OP, 2>), dim3(grid_of(r)), dim3(BLOCK), 0,
+        hipLaunchKernelGGL((k_stage<T, DIM, OP, 2>), dim3(grid_of(e, r)), dim3(BLOCK), 0,
                            e->stream, levels(e), st);
       } else
-        hipLaunchKernelGGL((k_stage<T, DIM, OP, 1>), dim3(grid_of(r)), dim3(BLOCK), 0,
+        hipLaunchKernelGGL((k_stage<T, DIM, OP, 1>), dim3(grid_of(e, r)), dim3(BLOCK), 0,
                            e->stream, levels(e), st);
     } else
-      hipLaunchKernelGGL((k_stage<T, DIM, OP, 0>), dim3(grid_of(r)), dim3(BLOCK), 0, e->stream,
+      hipLaunchKernelGGL((k_stage<T, DIM, OP, 0>), dim3(grid_of(e, r)), dim3(BLOCK), 0, e->stream,
                          levels(e), stage_of(e, r));
     if (probe) probe_end(e);
   }
@@ -805,18 +817,18 @@ struct Sched {
     if (r.nblocks == 0) return;
     if (mode == 2) {
       if (sweep)
-        hipLaunchKernelGGL((k_residual<T, DIM, true>), dim3(grid_of(*sweep)), dim3(BLOCK), 0,
+        hipLaunchKernelGGL((k_residual<T, DIM, true>), dim3(grid_of(e, *sweep)), dim3(BLOCK), 0,
                            e->stream, levels(e), stage_of(e, *sweep));
       else
-        hipLaunchKernelGGL((k_residual<T, DIM>), dim3(grid_of(fine)), dim3(BLOCK), 0,
+        hipLaunchKernelGGL((k_residual<T, DIM>), dim3(grid_of(e, fine)), dim3(BLOCK), 0,
                            e->stream, levels(e), stage_of(e, fine));
-      hipLaunchKernelGGL((k_restrict_gather<T, DIM>), dim3(grid_of(r)), dim3(BLOCK), 0,
+      hipLaunchKernelGGL((k_restrict_gather<T, DIM>), dim3(grid_of(e, r)), dim3(BLOCK), 0,
                          e->stream, levels(e), stage_of(e, r));
     } else if (mode == 1) {
-      hipLaunchKernelGGL((k_restrict_rows<T, DIM>), dim3(grid_of(r)), dim3(BLOCK), 0, e->stream,
+      hipLaunchKernelGGL((k_restrict_rows<T, DIM>), dim3(grid_of(e, r)), dim3(BLOCK), 0, e->stream,
                          levels(e), stage_of(e, r));
     } else {
-      hipLaunchKernelGGL((k_restrict<T, DIM>), dim3(grid_of(r)), dim3(BLOCK), 0, e->stream,
+      hipLaunchKernelGGL((k_restrict<T, DIM>), dim3(grid_of(e, r)), dim3(BLOCK), 0, e->stream,
                          levels(e), stage_of(e, r));
     }
   }
@@ -827,7 +839,8 @@ struct Sched {
                   bool levels = false, const Engine::StageRef& b = Engine::StageRef(),
                   CGState* out = nullptr) {
     if (r.n == 0) return;
-    const RunsPair rp{{{stage_of(e, a), grid_of(a), levels}, {stage_of(e, b), grid_of(b), false}}};
+    const RunsPair rp{{{stage_of(e, a), grid_of(e, a), levels},
+                       {stage_of(e, b), grid_of(e, b), false}}};
     hipLaunchKernelGGL((k_finalize<T, TX, OP>), dim3(r.n), dim3(BLOCK), 0, e->stream, sys(e),
                        (const Item*)(e->d_items + r.off), r.n, r.one, rp, out);
   }
@@ -850,10 +863,10 @@ struct Sched {
   // 5.83 -> 6.33, so it has two blocks per CU, where FP32 has three.
   static bool tiled(const Engine* e, int l) {
     const long n = e->st_tile[l].nblocks,
-               most = DIM == 2 ? 4l * g_tile_max
-                               : (sizeof(T) == 4 ? 1l * g_tile_max : 2l * g_tile_max / 3);
+               most = DIM == 2 ? 4l * e->kn.tile_max
+                               : (sizeof(T) == 4 ? 1l * e->kn.tile_max : 2l * e->kn.tile_max / 3);
     return n > 0 && n <= most && e->nu >= (DIM == 2 ? 1 : TILE_MAX_NU) && e->nu <= TILE_MAX_NU &&
-           g_fuse_first == 0 && g_fuse_prolong && restrict_mode_of(e, l) == 2 &&
+           e->kn.fuse_first == 0 && e->kn.fuse_prolong && restrict_mode_of(e, l) == 2 &&
            !(l == 0 && e->probe_on);  // the probe times level 0's half-sweeps
   }
 
@@ -865,7 +878,7 @@ struct Sched {
     for (int l = 0; l + 1 < L; ++l) {
       if (tiled(e, l)) {
         const Engine::StageRef& t = e->st_tile[l];
-        hipLaunchKernelGGL((k_tile_pre<T, DIM>), dim3(grid_of(t)), dim3(TileShape<DIM>::NT), 0,
+        hipLaunchKernelGGL((k_tile_pre<T, DIM>), dim3(grid_of(e, t)), dim3(TileShape<DIM>::NT), 0,
                            e->stream, levels(e), stage_of(e, t), nu);
         continue;
       }
@@ -874,7 +887,7 @@ struct Sched {
       // the last pre-smoothing smooth(l, 1) also forms the colour-1 residual
       // when the restriction is the two-pass one and that half-sweep exists
       const int rm = restrict_mode_of(e, l);
-      const bool ff = g_fuse_first == 1 || (g_fuse_first == 2 && l > 0);
+      const bool ff = e->kn.fuse_first == 1 || (e->kn.fuse_first == 2 && l > 0);
       const bool res1 = rm == 2 && nu > 0 && !(ff && nu == 1);
       if (nu > 0) {
         if (ff) {
@@ -932,11 +945,11 @@ struct Sched {
       if (tiled(e, l)) {
         const Engine::StageRef& t = e->st_tile[l];
         if (l == 0)
-          hipLaunchKernelGGL((k_tile_post<T, DIM, true>), dim3(grid_of(t)),
+          hipLaunchKernelGGL((k_tile_post<T, DIM, true>), dim3(grid_of(e, t)),
                              dim3(TileShape<DIM>::NT), 0, e->stream, levels(e), stage_of(e, t),
                              nu);
         else
-          hipLaunchKernelGGL((k_tile_post<T, DIM, false>), dim3(grid_of(t)),
+          hipLaunchKernelGGL((k_tile_post<T, DIM, false>), dim3(grid_of(e, t)),
                              dim3(TileShape<DIM>::NT), 0, e->stream, levels(e), stage_of(e, t),
                              nu);
         continue;
@@ -944,7 +957,7 @@ struct Sched {
       const Engine::StageRef& S = e->st_slot[l];
       const Engine::StageRef& W = e->st_sweep[l];
       if (nu > 0) {
-        if (g_fuse_prolong) {
+        if (e->kn.fuse_prolong) {
           stage<ST_PROLONG_SMOOTH1>(e, S, l == 0);
         } else {
           stage<ST_PROLONGATE0>(e, S, l == 0);
@@ -962,42 +975,43 @@ struct Sched {
     // level 0's last half-sweep fused with reduce(z, r) (its fused leg has
     // both), or a plain dot
     if (e->st_dot_fused.nblocks && !tiled(e, 0))
-      hipLaunchKernelGGL((k_smooth0_dot<T, TX, DIM>), dim3(grid_of(e->st_dot_fused)),
+      hipLaunchKernelGGL((k_smooth0_dot<T, TX, DIM>), dim3(grid_of(e, e->st_dot_fused)),
                          dim3(BLOCK), 0, e->stream, sys(e), stage_of(e, e->st_dot_fused));
     if (e->st_dot_plain.nblocks)
-      hipLaunchKernelGGL((k_dot_zr<T, TX>), dim3(grid_of(e->st_dot_plain)), dim3(BLOCK), 0,
+      hipLaunchKernelGGL((k_dot_zr<T, TX>), dim3(grid_of(e, e->st_dot_plain)), dim3(BLOCK), 0,
                          e->stream, sys(e), stage_of(e, e->st_dot_plain));
   }
 
   // One iteration for every member: the pre-loop of newly admitted systems
   // (mgpcg.py:157-172) and one loop body (:176-209) of the others.
   static void iteration(Engine* e, bool sync_each) {
+    e->kn = knobs_now();
     auto sync = [&]() {
       if (sync_each) (void)hipStreamSynchronize(e->stream);
     };
     if (e->st_init.nblocks) {
-      hipLaunchKernelGGL((k_cg_init<T, TX>), dim3(grid_of(e->st_init)), dim3(BLOCK), 0,
+      hipLaunchKernelGGL((k_cg_init<T, TX>), dim3(grid_of(e, e->st_init)), dim3(BLOCK), 0,
                          e->stream, sys(e), stage_of(e, e->st_init));
       fin<FIN_INIT>(e, e->fin_init, e->st_init);
       sync();
     }
     if (e->st_cg.nblocks) {
-      if (g_fuse_p) {
-        hipLaunchKernelGGL((k_cg_ap<T, TX, DIM>), dim3(grid_of(e->st_cg)), dim3(BLOCK), 0,
+      if (e->kn.fuse_p) {
+        hipLaunchKernelGGL((k_cg_ap<T, TX, DIM>), dim3(grid_of(e, e->st_cg)), dim3(BLOCK), 0,
                            e->stream, sys(e), stage_of(e, e->st_cg));
       } else {
-        hipLaunchKernelGGL((k_cg_update_p<T, TX>), dim3(grid_of(e->st_cg)), dim3(BLOCK), 0,
+        hipLaunchKernelGGL((k_cg_update_p<T, TX>), dim3(grid_of(e, e->st_cg)), dim3(BLOCK), 0,
                            e->stream, sys(e), stage_of(e, e->st_cg));
-        hipLaunchKernelGGL((k_cg_ap_only<T, TX, DIM>), dim3(grid_of(e->st_cg)), dim3(BLOCK), 0,
+        hipLaunchKernelGGL((k_cg_ap_only<T, TX, DIM>), dim3(grid_of(e, e->st_cg)), dim3(BLOCK), 0,
                            e->stream, sys(e), stage_of(e, e->st_cg));
       }
       fin<FIN_ALPHA>(e, e->fin_cg, e->st_cg);
       sync();
-      hipLaunchKernelGGL((k_cg_xr<T, TX>), dim3(grid_of(e->st_cg)), dim3(BLOCK), 0, e->stream,
+      hipLaunchKernelGGL((k_cg_xr<T, TX>), dim3(grid_of(e, e->st_cg)), dim3(BLOCK), 0, e->stream,
                          sys(e), stage_of(e, e->st_cg));
       fin<FIN_RR>(e, e->fin_cg, e->st_cg);
       if (e->precision == MIXED) {
-        hipLaunchKernelGGL((k_true_residual<T, TX, DIM>), dim3(grid_of(e->st_cg)), dim3(BLOCK),
+        hipLaunchKernelGGL((k_true_residual<T, TX, DIM>), dim3(grid_of(e, e->st_cg)), dim3(BLOCK),
                            0, e->stream, sys(e), stage_of(e, e->st_cg));
         fin<FIN_TRUE>(e, e->fin_cg, e->st_cg);
       }
@@ -1049,6 +1063,7 @@ struct RunGather {
 template <typename T, typename TX, int DIM>
 struct RunVcycle {
   static int run(Engine* e) {
+    e->kn = knobs_now();
     Sched<T, TX, DIM>::vcycle(e);
     return 0;
   }
@@ -1890,6 +1905,7 @@ struct RefPath {
   static int run(Engine* e, mgpcg_solver* s, int max_iters, double rel_tol, double abs_tol,
                  double eps, mgpcg_result_t* out) {
     using Sd = Sched<T, TX, DIM>;
+    e->kn = knobs_now();
     const int L = s->L, nu = s->nu;
     const SysDesc<T, TX>* sysd = Sd::sys(e);
     const LevelDesc<T>* lv = Sd::levels(e);
@@ -2140,7 +2156,7 @@ template <typename T, typename TX, int DIM>
 struct RunOp {
   static int run(Engine* e, int op, const Engine::StageRef& r, int arg, bool level0) {
     using Sd = Sched<T, TX, DIM>;
-    const int nb = r.nblocks;
+    e->kn = knobs_now();
     switch (op) {
       case MGPCG_OP_SMOOTH:
         if (arg & 1) Sd::template stage<ST_SMOOTH1>(e, r, level0);
@@ -2162,7 +2178,7 @@ struct RunOp {
         Sd::template stage<ST_PROLONGATE>(e, r);
         return 0;
       case MGPCG_OP_COMPUTE_AP:
-        hipLaunchKernelGGL((k_cg_ap<T, TX, DIM>), dim3(std::min(nb, g_max_grid)), dim3(BLOCK), 0,
+        hipLaunchKernelGGL((k_cg_ap<T, TX, DIM>), dim3(grid_of(e, r)), dim3(BLOCK), 0,
                            e->stream, Sd::sys(e), stage_of(e, r));
         return 0;
       default:

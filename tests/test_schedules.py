@@ -94,3 +94,49 @@ def test_dot_products_at_block_counts(dev, res, blocks, L):
     xr, outr, _ = osys.solve(sysd, core.PLAIN, max_iters=4, rel_tol=1e-12)
     assert out["iters"] == outr["iters"]
     assert np.array_equal(x, xr)
+
+
+def test_options_changed_by_another_thread_during_a_solve(dev):
+    """The options are process-wide and a solve may run while another thread
+    sets them: each iteration keeps those it began with, and the bits are the
+    oracle's whatever they are."""
+    import threading
+
+    from mgpcg_amd import _lib, mgpcg, systems
+
+    lib = _lib.load()
+    sysd = scenes.pool_sphere_system([62, 50], 9, L=2, kind="pressure")
+    xr, outr, _ = osys.solve(sysd, core.PLAIN, max_iters=8, rel_tol=1e-12)
+    d = systems.upload(sysd, dev)
+    set_knobs(coarse_max=0)
+    solvers = [mgpcg.MGPCGPoissonSolver(2, sysd["res"], 2, sysd["nu"], sysd["bottom"], device=dev)
+               for _ in range(3)]
+    stop = threading.Event()
+    changes = [0]
+
+    def change():
+        rng = np.random.default_rng(1)
+        values = [(_lib.OPT_MAX_GRID, (8, 9, 2048)), (_lib.OPT_TILE_MAX, (0, 768)),
+                  (_lib.OPT_FUSE_PROLONG, (0, 1)), (_lib.OPT_FUSE_FIRST, (0, 1)),
+                  (_lib.OPT_FUSE_P, (0, 1))]
+        while not stop.is_set():
+            option, of = values[rng.integers(len(values))]
+            _lib.check(lib.mgpcg_set_option(None, option, int(of[rng.integers(len(of))])))
+            changes[0] += 1
+
+    t = threading.Thread(target=change)
+    t.start()
+    try:
+        for i in range(12):
+            s = solvers[i % 3]
+            systems.assemble(s, d)
+            s.solve(8, rel_tol=1e-12)
+            _lib.synchronize(dev)
+            assert s.last["iters"] == outr["iters"], (i, changes[0])
+            assert np.array_equal(_x(s), xr), (i, changes[0])
+    finally:
+        stop.set()
+        t.join()
+        set_knobs(**KNOB_DEFAULTS)
+        _tile_max(768)
+    assert changes[0] > 10
