@@ -380,9 +380,10 @@ int mgpcg_redistance(void* stream, int dim, const int32_t* res, double dx, int r
  * place: per component, faces next to a FLUID cell are valid; `iterations`
  * (10 in the reference) passes average the valid faces of each invalid face's
  * 3^dim neighbourhood into it.  backup (floats), valid and valid_temp (bytes)
- * are work arrays of at least the largest component's size (backup alone is
- * written: it holds the flags, a bit per face).  Faces outside a component's
- * shape count as invalid. */
+ * are work arrays of at least the largest component's size, none of them NULL;
+ * backup alone is used (it holds the flags, a bit per face), so valid and
+ * valid_temp may be any address.  Faces outside a component's shape count as
+ * invalid. */
 int mgpcg_extrap_velocity(void* stream, int dim, const int32_t* res, const int8_t* cell_type,
                           float* const* velocity, int iterations, float* backup, int8_t* valid,
                           int8_t* valid_temp);

@@ -56,9 +56,8 @@ def extrap_velocity(velocity, cell_type, iterations=10):
     dev = cell_type.device
     n = max(u.numel() for u in velocity)
     backup = torch.empty(n, dtype=torch.float32, device=dev)
-    valid = torch.empty(n, dtype=torch.int8, device=dev)
-    valid_temp = torch.empty(n, dtype=torch.int8, device=dev)
+    # the two byte arrays of the interface are not used: the flags are bits in backup
     _lib.check(lib.mgpcg_extrap_velocity(
         _lib.stream_handle(dev), dim, _lib.int3(res), _lib.ptr(cell_type), _vel_ptrs(velocity),
-        int(iterations), _lib.ptr(backup), _lib.ptr(valid), _lib.ptr(valid_temp)))
+        int(iterations), _lib.ptr(backup), _lib.ptr(backup), _lib.ptr(backup)))
 
